@@ -1,20 +1,27 @@
 // kb_blk_impl.h -- blocked batched Cholesky family, one 256-thread workgroup
 // per matrix, for orders above the register-resident range.
 //
-// Right-looking blocked algorithm with panel width NBK = 32, the same
-// POTRF -> TRSM(R,L,T) -> SYRK(L,N,-1,+1) sequence the reference runs as a
-// recursion of separate launches (src/batch_triangular/Xpotrf_batch_drivers.cuh:91-131),
-// here inside one kernel so every stage of a matrix reuses the workgroup's
-// LDS and the matrix's cache lines:
-//   - the 32x32 diagonal block is factored by wave 0 in registers as three
-//     16x16 tiles (4-column panels on DPP rows, rank-4 updates on the matrix
-//     cores), written to memory and to LDS with its inverse diagonal;
-//   - the panel below is solved one row per thread against the LDS block;
-//   - panels go in pairs: the second panel's columns are updated with the
-//     first, and the trailing lower triangle then receives one update of
-//     depth 64 (both panels) on the matrix cores, in 64x64 tiles (one 64x64
-//     slice staged in LDS, the other operand in registers), so the trailing
-//     matrix is read and written once per 64 columns instead of once per 32.
+// Left-looking blocked algorithm with panel width NBK = 32, the same POTRF ->
+// TRSM(R,L,T) -> SYRK(L,N,-1,+1) arithmetic the reference runs as a recursion
+// of separate launches (src/batch_triangular/Xpotrf_batch_drivers.cuh:91-131),
+// here inside one kernel.  Per panel (blk_potrf below):
+//   - wave 0 reads the 32x32 diagonal block as three 16x16 tiles, subtracts
+//     the products of the finished columns on the matrix cores, factors it in
+//     registers (4-column panels on DPP rows, rank-4 updates on the matrix
+//     cores) and leaves the inverses of the two 16x16 diagonal tiles in LDS;
+//   - meanwhile waves 1..3 read the 16-row tiles below and subtract the same
+//     products, then solve them against the inverses, all in registers: every
+//     element of A is read once and every element of L written once, and the
+//     only other traffic is re-reading finished columns of L;
+//   - right-hand sides (POSV) are further row tiles of the panel: the forward
+//     sweep L Y = B is the panel solve Y^T = B^T L^-T.
+// What bounds it: the serial chain of a panel (the loads' latency, the 32
+// pivots, two barriers), hidden by four workgroups per CU.  Against the
+// right-looking form it replaces (trailing matrix read and written once per 64
+// columns, rows solved by substitution one per thread): DPOTRF n = 200 x 2,000
+// 725 -> 350 us, n = 256 x 4,096 1.82 -> 0.86 ms, n = 128 x 8,000 0.82 -> 0.45
+// ms; the workgroup phase of the non-uniform DPOSV of orders 8..256 x 20,000
+// 4.50 -> 2.65 ms.
 // The solve (POSV/POTRS) runs blocked forward and backward sweeps over up to
 // 64 right-hand sides per pass (so L is streamed once per sweep for up to 64
 // right-hand sides): the diagonal blocks by DPP-row substitutions, the
@@ -27,21 +34,28 @@
 #include "kb_tile_impl.h"
 
 constexpr int KB_BLK_NBK = 32;
-constexpr int KB_BLK_KW = 2 * KB_BLK_NBK;   // depth of a trailing update (two panels)
 constexpr int KB_BLK_WG = 256;
-constexpr int KB_BLK_TILE = 64;
 constexpr int KB_BLK_RC = 64;   // right-hand sides per pass of the solve
+constexpr int KB_LL_LD = 17;    // pitch of a staged 16 x 16 tile
+// 16-row tiles a wave holds at once (C and the running sums: FP64 16 VGPRs each
+// per tile).  FP64: 2 fill the 128 VGPRs that four workgroups per CU leave; 3
+// spill there, and with three workgroups per CU n = 128 takes 0.61 instead of
+// 0.45 ms.  FP32: 4 against 2 is n = 200 x 4,000 0.57 against 0.63 ms.
+template <typename T> constexpr int ll_g();
+template <> constexpr int ll_g<double>() { return 2; }
+template <> constexpr int ll_g<float>() { return 4; }
 
-// The trailing update's staged slice is never live at the same time as the
-// diagonal block, the panel transposes or the solve's staging, so they share
-// its space (33 KB for FP64 instead of 44 KB).
+// The factorization's blocks and the solve's staging are never live together.
 template <typename T>
 struct BlkSmem {
     union {
-        T sB[KB_BLK_TILE * (KB_BLK_KW + 1)];   // a 64-row slice of the panels (trailing update)
         struct {
             T sY[KB_BLK_RC * (KB_BLK_NBK + 1)];   // the solve's staging of a block of the solution
             T sD[KB_BLK_NBK * (KB_BLK_NBK + 1)];  // the diagonal block
+        };
+        struct {
+            T fD[KB_BLK_NBK * (KB_BLK_NBK + 1)];  // the factored diagonal block
+            T fW[2][16 * KB_LL_LD];               // the inverses of its diagonal 16 x 16 tiles
             T tpan[4][16][4];                     // panel transposes of the diagonal-block factorization
         };
     };
@@ -54,76 +68,6 @@ template <typename T>
 KB_DEV T& rhs_at(T* B, int ldb, int side_left, int i, int c)
 {
     return side_left ? B[i + (long)c * ldb] : B[c + (long)i * ldb];
-}
-
-// C (m2 x m2, lower; only its first ncol columns) -= L21 L21^T, L21 is
-// m2 x kb (kb <= 64, ld lda), on the matrix cores.  C is walked in 64 x 64
-// tiles.  Wave w computes rows 16w..16w+15 of a tile as four 16 x 16 products
-// D' = L21_J(16 x kb) L21_I(16 x kb)^T, i.e. the transpose of the C block,
-// whose accumulator layout puts consecutive C rows in consecutive lanes
-// (coalesced column-major read-modify-write):
-//   FP64: lane (g, i), register r -> C(16w + i, 16q + 4r + g)
-//   FP32: lane (g, i), register r -> C(16w + i, 16q + 4g + r)
-// The wave's own 16 rows of slice I (the B operand of every K step) stay in
-// registers for the whole row of tiles; slice J is staged in LDS.
-template <typename T>
-KB_DEV void blk_syrk_update(const T* L21, T* C, int lda, int m2, int kb, BlkSmem<T>& S, int ncol)
-{
-    constexpr int KW = KB_BLK_KW, TL = KB_BLK_TILE;
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));   // lane-dependent values formed per call, not kept live across
-    const int wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, lg = lane >> 4;
-    const int nt = (m2 + TL - 1) / TL;
-    const int kb4 = (kb + 3) & ~3;
-    for (int I = 0; I < nt; ++I) {
-        const int gi = I * TL + 16 * wave + li;
-        T bI[KW / 4];
-#pragma unroll
-        for (int u = 0; u < KW / 4; ++u) {
-            const int p = 4 * u + lg;
-            const bool in = gi < m2 && p < kb;
-            const T v = gld(L21 + (in ? gi + (long)p * lda : 0));
-            bI[u] = in ? v : T(0);
-        }
-        for (int J = 0; J <= I && J * TL < ncol; ++J) {
-            for (int e = tid; e < TL * KW; e += KB_BLK_WG) {
-                const int r = e % TL, p = e / TL;
-                const int gj = J * TL + r;
-                if (p < kb4) S.sB[r * (KW + 1) + p] = (gj < m2 && p < kb) ? gld(L21 + gj + (long)p * lda) : T(0);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (J == I && q > wave) continue;          // above the diagonal
-                if (J * TL + 16 * q >= ncol) continue;     // beyond the columns asked for
-                int col[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    col[r] = J * TL + 16 * q + ((sizeof(T) == 8) ? 4 * r + lg : 4 * lg + r);
-                // the C block first, so its latency overlaps the products
-                T cv[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const bool in = gi < m2 && col[r] <= gi && col[r] < ncol;
-                    const T v = gld(C + (in ? gi + (long)col[r] * lda : 0));
-                    cv[r] = in ? v : T(0);
-                }
-                typename TileV<T>::v4 acc = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-                for (int u = 0; u < KW / 4; ++u) {
-                    if (4 * u < kb) {
-                        const T a = S.sB[(16 * q + li) * (KW + 1) + 4 * u + lg];
-                        acc = mfma16x16x4(a, bI[u], acc);
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (gi < m2 && col[r] <= gi && col[r] < ncol) gst(C + gi + (long)col[r] * lda, cv[r] - acc[r]);
-            }
-            __syncthreads();
-        }
-    }
 }
 
 // The diagonal block L(k0.., k0..) of the factor in two steps, so the solve
@@ -162,92 +106,6 @@ KB_DEV void blk_diag_put(const T (&v)[KB_BLK_DPT], int kb, BlkSmem<T>& S, int un
         if (r == c) S.sInv[r] = (r < kb && !unit) ? T(1) / v[m] : T(1);
     }
     __syncthreads();
-}
-
-// One 32-column panel at k0 (kb columns, already updated by every panel to
-// its left): its diagonal block factored by wave 0 (L_D also goes to LDS for
-// the panel solve), then the rows below solved one row per thread,
-// X L_D^T = A_panel.  Returns LAPACK info (0, or k0 + the failing column).
-template <typename T>
-KB_DEV int blk_panel(T* A, int lda, int n, int k0, int kb, BlkSmem<T>& S)
-{
-    constexpr int NBK = KB_BLK_NBK;
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));   // lane-dependent values formed per panel, not kept live across
-    const int wave = tid >> 6, lane = tid & 63;
-    if (wave == 0) {
-        // the 32 x 32 diagonal block as tiles (0,0), (1,0), (1,1): lane (i, g)
-        // holds row i and columns 4g..4g+3 of each; rows and columns at or
-        // beyond kb read as the identity
-        T* D = A + k0 + (long)k0 * lda;
-        const int i = lane & 15, g = lane >> 4;
-        typename TileV<T>::v4 td[3];
-#pragma unroll
-        for (int I = 0; I < 2; ++I)
-#pragma unroll
-            for (int J = 0; J <= I; ++J)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 16 * I + i, col = 16 * J + 4 * g + r;
-                    const bool in = row < kb && col <= row;
-                    const T v = gld(D + (in ? row + (long)col * lda : 0));
-                    td[tix(I, J)][r] = in ? v : ((row == col) ? T(1) : T(0));
-                }
-        T invd[2] = {T(1), T(1)};
-        const int inf = tile_potrf<T, 2>(td, invd, kb, S.tpan, lane);
-        // L_D to memory (lower part), to LDS for the panel solve below, and
-        // 1/L(j, j) to sInv
-#pragma unroll
-        for (int I = 0; I < 2; ++I)
-#pragma unroll
-            for (int J = 0; J <= I; ++J)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 16 * I + i, col = 16 * J + 4 * g + r;
-                    if (row < kb && col <= row) gst(D + row + (long)col * lda, td[tix(I, J)][r]);
-                    S.sD[row * (NBK + 1) + col] = (col <= row) ? td[tix(I, J)][r] : T(0);
-                }
-        if (g == 0) {
-            S.sInv[i] = invd[0];
-            S.sInv[16 + i] = invd[1];
-        }
-        if (lane == 0) S.flag = inf ? k0 + inf : 0;
-    }
-    __syncthreads();
-    const int f = S.flag;
-    if (f) return f;
-    for (int i = k0 + kb + tid; i < n; i += KB_BLK_WG) {
-        T x[NBK];
-        // walk the row with a running pointer (made opaque each step), so the
-        // 32 column addresses are not precomputed and kept live across rows
-        T* p = A + i + (long)k0 * lda;
-#pragma unroll
-        for (int c = 0; c < NBK; ++c) {
-            x[c] = (c < kb) ? gld(p) : T(0);
-            p += lda;
-            asm volatile("" : "+v"(p));
-        }
-#pragma unroll
-        for (int j = 0; j < NBK; ++j) {
-            if (j < kb) {
-                x[j] = x[j] * S.sInv[j];
-#pragma unroll
-                for (int c = j + 1; c < NBK; ++c) x[c] = kb_fma<T>(-x[j], S.sD[c * (NBK + 1) + j], x[c]);
-            }
-            // keep each step's LDS reads with the step (hoisting them all would
-            // spill the 32-element row)
-            asm volatile("" ::: "memory");
-        }
-        p = A + i + (long)k0 * lda;
-#pragma unroll
-        for (int c = 0; c < NBK; ++c) {
-            if (c < kb) gst(p, x[c]);
-            p += lda;
-            asm volatile("" : "+v"(p));
-        }
-    }
-    __syncthreads();
-    return 0;
 }
 
 // Row of a 16x16 matrix-core accumulator held in register q by lanes 16g..16g+15
@@ -498,34 +356,344 @@ KB_DEV void blk_solve(const T* L, int lda, int n, T* B, int ldb, int side_left, 
     blk_solve_bwd<T, CB>(L, lda, n, B, ldb, side_left, nrhs, S);
 }
 
+// ---------------------------------------------------------------------------
+// factorization
+// ---------------------------------------------------------------------------
+// A 16-row tile of the panel: element (row i of the tile, column k) at
+// p + i * rs + k * cs.  Rows of A: (rs, cs) = (1, lda); right-hand sides
+// (row i is right-hand side i): (1, ldb) for side right, (ldb, 1) for left.
+template <typename T>
+struct LlTile {
+    T* p;
+    long rs, cs;
+    int rows;   // valid rows (1..16)
+};
+
+// Columns between a lane's accumulator elements e and e + 1 of a tile.
+template <typename T> constexpr int ll_step(int e) { return sizeof(T) == 8 ? 4 : (e & 3) == 3 ? 13 : 1; }
+
+// K steps of 4 columns whose loads go out together (a second set is in flight
+// while they are multiplied).
+constexpr int KB_LL_U = 1;
+constexpr int KB_LL_KC = 64;   // columns whose products are summed before they are taken from C
+
+// c[j] := C_j - L_j L_P^T in transposed form for NT tiles: register r of column
+// block q holds, in lane (i, g), row i and panel column 16 q + blk_drow(r, g).
+// Lp: the panel's rows of L (row k0, column 0), kb of them valid; rows and
+// columns beyond the valid ones repeat the last (their results are never
+// used).  The products of 64 columns at a time are summed by themselves and
+// then taken from C: added to C one by one they would each be rounded at its
+// size, and a sum over all the columns at the size of the whole sum.
+template <typename T, int NT>
+KB_DEV void ll_update(const T* Lp, int lda, int kb, int k0, const LlTile<T>* t, int li, int lg,
+                      typename TileV<T>::v4 (&c)[NT][2])
+{
+    typedef typename TileV<T>::v4 v4;
+    // formed here, not kept live (or as induction variables) across panels
+    asm volatile("" : "+v"(li), "+v"(lg));
+    asm volatile("" : "+s"(k0));
+    constexpr int U = KB_LL_U;
+    const T* pb[NT];
+    const T* pa[2];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const T* p = t[j].p + (long)min(li, t[j].rows - 1) * t[j].rs;
+        pb[j] = p + lg * t[j].cs;
+        // a running pointer (opaque each step), so the column addresses are not
+        // all formed at once; it stops at the last valid column
+        p += (k0 + min(blk_drow<T>(0, lg), kb - 1)) * t[j].cs;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            c[j][e >> 2][e & 3] = gld(p);
+            if (16 * ((e + 1) >> 2) + blk_drow<T>((e + 1) & 3, lg) < kb) p += ll_step<T>(e) * t[j].cs;
+            asm volatile("" : "+v"(p));
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) pa[q] = Lp + min(16 * q + li, kb - 1) + (long)lg * lda;
+    T a[U][2], b[U][NT], an[U][2], bn[U][NT];
+    auto fetch = [&](T (&xa)[U][2], T (&xb)[U][NT]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                xa[u][q] = gld(pa[q]);
+                pa[q] += 4 * (long)lda;
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                xb[u][j] = gld(pb[j]);
+                pb[j] += 4 * t[j].cs;
+            }
+        }
+    };
+    v4 acc[NT][2];
+    auto mult = [&](const T (&xa)[U][2], const T (&xb)[U][NT]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[j][q] = mfma16x16x4(xa[u][q], xb[u][j], acc[j][q]);
+    };
+    if (k0 > 0) fetch(a, b);
+    for (int kc = 0; kc < k0; kc += KB_LL_KC) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j][0] = acc[j][1] = v4{T(0), T(0), T(0), T(0)};
+        // k0 and KB_LL_KC are multiples of 32, so the steps come in pairs of U
+        const int ke = min(kc + KB_LL_KC, k0);
+        for (int k = kc; k < ke; k += 8 * U) {
+            fetch(an, bn);
+            mult(a, b);
+            __builtin_amdgcn_sched_barrier(0);
+            if (k + 8 * U < k0) fetch(a, b);
+            mult(an, bn);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) c[j][q] -= acc[j][q];
+    }
+}
+
+// W c for the inverse W of a 16 x 16 triangle
+template <typename T>
+KB_DEV typename TileV<T>::v4 ll_apply(const T* W, int li, int lg, const typename TileV<T>::v4& c)
+{
+    typename TileV<T>::v4 x = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x = mfma16x16x4(W[li * KB_LL_LD + blk_drow<T>(s, lg)], c[s], x);
+    return x;
+}
+
+// One updated tile solved against the factored diagonal block and stored:
+// X1^T = L11^-1 C1^T, X2^T = L22^-1 (C2^T - L21 X1^T).  A 16 x 16 accumulator is
+// itself the second operand of the next product (register s of lane group g
+// holds row kmap(s, g)), so nothing leaves the registers.
+template <typename T>
+KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const BlkSmem<T>& S,
+                     typename TileV<T>::v4 (&c)[2])
+{
+    constexpr int LD = KB_BLK_NBK + 1;
+    typename TileV<T>::v4 x[2];
+    if (kb < KB_BLK_NBK) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (16 * (e >> 2) + blk_drow<T>(e & 3, lg) >= kb) c[e >> 2][e & 3] = T(0);
+    }
+    x[0] = ll_apply<T>(S.fW[0], li, lg, c[0]);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c[1] = mfma16x16x4(-S.fD[(16 + li) * LD + blk_drow<T>(s, lg)], x[0][s], c[1]);
+    x[1] = ll_apply<T>(S.fW[1], li, lg, c[1]);
+    T* p = t.p + (long)li * t.rs + (k0 + blk_drow<T>(0, lg)) * t.cs;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if (li < t.rows && 16 * (e >> 2) + blk_drow<T>(e & 3, lg) < kb) gst(p, x[e >> 2][e & 3]);
+        p += ll_step<T>(e) * t.cs;
+        asm volatile("" : "+v"(p));
+    }
+}
+
+// One wave's NT tiles of a panel: update, wait for the diagonal block (first:
+// every wave of the workgroup passes exactly one barrier here, in ll_diag's
+// branch or in one of these), solve.  Returns S.flag.
+template <typename T, int NT>
+KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTile<T>* t, int li, int lg,
+                    const BlkSmem<T>& S)
+{
+    typename TileV<T>::v4 c[NT > 0 ? NT : 1][2];
+    if constexpr (NT > 0) ll_update<T, NT>(Lp, lda, kb, k0, t, li, lg, c);
+    if (first) {
+        __syncthreads();
+        const int f = S.flag;
+        if (f) return f;
+    }
+    if constexpr (NT > 0) {
+        // formed here, not kept live (or as induction variables) across panels
+        asm volatile("" : "+v"(li), "+v"(lg));
+        asm volatile("" : "+s"(k0));
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            ll_solve<T>(t[j], kb, k0, li, lg, S, c[j]);
+            __builtin_amdgcn_sched_barrier(0);   // one tile's products at a time (registers)
+        }
+    }
+    return 0;
+}
+
+// Wave 0's part of a panel: the diagonal block (k0, kb) updated with the k0
+// finished columns, factored, written to memory and to LDS with the inverses
+// of its two 16 x 16 diagonal tiles.  S.flag: 0 or k0 + the failing
+// column (1-based).
+template <typename T>
+KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
+{
+    constexpr int LD = KB_BLK_NBK + 1;
+    asm volatile("" : "+v"(lane));
+    asm volatile("" : "+s"(k0));
+    const int i = lane & 15, g = lane >> 4;
+    const int ci = (sizeof(T) == 8) ? 4 * (i & 3) + (i >> 2) : i;   // as in tile_potrf
+    T* D = A + k0 + (long)k0 * lda;
+    const T* Lp = A + k0;
+    typename TileV<T>::v4 td[3];
+#pragma unroll
+    for (int I = 0; I < 2; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * I + i, col = 16 * J + 4 * g + r;
+                td[tix(I, J)][r] = gld(D + ((row < kb && col <= row) ? row + (long)col * lda : 0));
+            }
+    const T *pa[2], *pb[2];
+#pragma unroll
+    for (int I = 0; I < 2; ++I) {
+        pa[I] = Lp + min(16 * I + ci, kb - 1) + (long)g * lda;
+        pb[I] = Lp + min(16 * I + i, kb - 1) + (long)g * lda;
+    }
+    for (int kc = 0; kc < k0; kc += KB_LL_KC) {   // as in ll_update
+        typename TileV<T>::v4 acc[3];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) acc[x] = typename TileV<T>::v4{T(0), T(0), T(0), T(0)};
+        const int ke = min(kc + KB_LL_KC, k0);
+        for (int k = kc; k < ke; k += 16) {
+            T a[4][2], b[4][2];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int I = 0; I < 2; ++I) {
+                    a[u][I] = gld(pa[I]);
+                    b[u][I] = gld(pb[I]);
+                    pa[I] += 4 * (long)lda;
+                    pb[I] += 4 * (long)lda;
+                }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                acc[0] = mfma16x16x4(a[u][0], b[u][0], acc[0]);
+                acc[1] = mfma16x16x4(a[u][0], b[u][1], acc[1]);
+                acc[2] = mfma16x16x4(a[u][1], b[u][1], acc[2]);
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < 3; ++x) td[x] -= acc[x];
+    }
+    // rows and columns at or beyond kb, and the upper triangle, read as the identity
+#pragma unroll
+    for (int I = 0; I < 2; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * I + i, col = 16 * J + 4 * g + r;
+                if (!(row < kb && col <= row)) td[tix(I, J)][r] = (row == col) ? T(1) : T(0);
+            }
+    T invd[2] = {T(1), T(1)};
+    const int inf = tile_potrf<T, 2>(td, invd, kb, S.tpan, lane);
+#pragma unroll
+    for (int I = 0; I < 2; ++I)
+#pragma unroll
+        for (int J = 0; J <= I; ++J)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * I + i, col = 16 * J + 4 * g + r;
+                if (row < kb && col <= row) gst(D + row + (long)col * lda, td[tix(I, J)][r]);
+                S.fD[row * LD + col] = (col <= row) ? td[tix(I, J)][r] : T(0);
+            }
+    if (g == 0) {
+        S.sInv[i] = invd[0];
+        S.sInv[16 + i] = invd[1];
+    }
+    if (lane == 0) S.flag = inf ? k0 + inf : 0;
+    wave_lds_sync();
+    // the inverses of both diagonal tiles: DPP row g takes columns 4g..4g+3 of
+    // each, lane i of the row holds their row i
+    T y[2][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) y[0][s] = y[1][s] = (i == 4 * g + s) ? T(1) : T(0);
+#pragma unroll
+    for (int j = 0; j < 15; ++j) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const T ij = S.sInv[16 * b + j];
+            const T l = (i > j) ? S.fD[(16 * b + i) * LD + 16 * b + j] : T(0);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) fnmac_rowk<T>(y[b][s], y[b][s] * ij, l, j);
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) S.fW[b][i * KB_LL_LD + 4 * g + s] = y[b][s] * S.sInv[16 * b + i];
+}
+
 // In-place lower Cholesky of an n x n matrix by the whole workgroup.
 // Returns LAPACK info (identical in every thread).  With B given (POSV), the
-// forward sweep L Y = B runs inside the factorization: each panel's block step
-// follows the panel, while its diagonal block is still in LDS and the panel
-// in cache; a factorization that fails at panel k leaves B forward-solved
-// through the panels before k.
+// forward sweep L Y = B runs inside the factorization, the right-hand sides
+// being further row tiles of every panel; a factorization that fails at panel k
+// leaves B forward-solved in the rows of the panels before k and as it was in
+// the others.
 template <typename T, int CB = 4>
 KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ldb = 0, int side_left = 0,
                      int nrhs = 0)
 {
-    constexpr int NBK = KB_BLK_NBK;
-    for (int k0 = 0; k0 < n; k0 += 2 * NBK) {
-        const int kb0 = min(NBK, n - k0);
-        int f = blk_panel<T>(A, lda, n, k0, kb0, S);
-        if (f) return f;
-        if (B) blk_fwd_step<T, CB>(A, lda, n, k0, kb0, B, ldb, side_left, nrhs, S);
-        const int k1 = k0 + kb0;
-        if (k1 >= n) break;
-        const int kb1 = min(NBK, n - k1);
-        // the second panel's columns, updated with the first
-        blk_syrk_update<T>(A + k1 + (long)k0 * lda, A + k1 + (long)k1 * lda, lda, n - k1, kb0, S, kb1);
-        __syncthreads();
-        f = blk_panel<T>(A, lda, n, k1, kb1, S);
-        if (f) return f;
-        if (B) blk_fwd_step<T, CB>(A, lda, n, k1, kb1, B, ldb, side_left, nrhs, S);
-        // the trailing matrix, with both panels at once (depth kb0 + kb1)
-        const int t0 = k1 + kb1;
-        if (t0 < n) blk_syrk_update<T>(A + t0 + (long)k0 * lda, A + t0 + (long)t0 * lda, lda, n - t0, kb0 + kb1, S, n - t0);
+    constexpr int NBK = KB_BLK_NBK, G = ll_g<T>(), NW = KB_BLK_WG / 64;
+    static_assert(G <= 4, "one case per tile count below");
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // lane-dependent values formed per call, not kept live across
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int li = lane & 15, lg = lane >> 4;
+    const int nrt = B ? (nrhs + 15) >> 4 : 0;
+    for (int k0 = 0; k0 < n; k0 += NBK) {
+        const int kb = min(NBK, n - k0);
+        const int nt = max((n - k0 - NBK + 15) >> 4, 0);   // row tiles below the diagonal block
+        const int rest = nt + nrt;
+        auto tile = [&](int q) {   // tile q of the panel: rows of A, then right-hand sides
+            LlTile<T> t;
+            if (q < nt) {
+                const int r0 = k0 + NBK + 16 * q;
+                t.p = A + r0;
+                t.rs = 1;
+                t.cs = lda;
+                t.rows = min(16, n - r0);
+            } else {
+                const int c0 = 16 * (q - nt);
+                t.rs = side_left ? ldb : 1;
+                t.cs = side_left ? 1 : ldb;
+                t.p = B + c0 * t.rs;
+                t.rows = min(16, nrhs - c0);
+            }
+            return t;
+        };
+        // rounds of up to G tiles per wave; in the first, wave 0 factors the
+        // diagonal block instead, and nothing is solved before that is done
+        for (int base = 0, nw = NW - 1; base < rest || nw == NW - 1; nw = NW) {
+            const int round = min(rest - base, nw * G);
+            const int per = (round + nw - 1) / nw;
+            const int q0 = base + (wave - NW + nw) * per;
+            const int cnt = (q0 < base) ? 0 : max(min(per, base + round - q0), 0);
+            const bool diag = nw == NW - 1;
+            LlTile<T> t[G];
+#pragma unroll
+            for (int j = 0; j < G; ++j) t[j] = tile(max(min(q0 + j, rest - 1), 0));
+            int f;
+            if (diag && wave == 0) {
+                ll_diag<T>(A, lda, k0, kb, S, lane);
+                f = ll_group<T, 0>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            } else if (G >= 4 && cnt == 4) {
+                f = ll_group<T, G >= 4 ? 4 : 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            } else if (G >= 3 && cnt == 3) {
+                f = ll_group<T, G >= 3 ? 3 : 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            } else if (cnt == 2) {
+                f = ll_group<T, 2>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            } else if (cnt == 1) {
+                f = ll_group<T, 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            } else {
+                f = ll_group<T, 0>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+            }
+            if (f) return f;
+            base += round;
+        }
         __syncthreads();
     }
     return 0;

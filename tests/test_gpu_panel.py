@@ -1,0 +1,91 @@
+"""GPU parity tests of the workgroup Cholesky (orders above 64) at the edges of
+its panels, against the oracle (orc_posv): orders at and around multiples of
+the 16-row tiles and 32-column panels, orders whose panels need a second round
+of row tiles (above 32 + 12 * 16 = 224 rows, fewer with right-hand sides), and
+right-hand-side counts at and around 16 (they are further row tiles of every
+panel), both sides, both precisions, strided and pointer-array operands.
+
+Bar: the factor's and the solution's normwise backward errors <= 4 n eps, the
+solution within 64 n eps of the oracle's (max-norm, relative to max(|X|, 1)).
+One matrix is not positive definite: LAPACK's info, its neighbours unharmed.
+The strict upper triangle holds NaN and is never read or written, padding rows
+of A and B are never written."""
+import numpy as np
+import pytest
+
+import kbtest as kt
+import pykblas
+import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def h():
+    hh = kt.handle()
+    yield hh
+    hh.close()
+
+
+CASES = [(65, 1), (79, 16), (80, 17), (81, 33), (96, 0), (97, 4), (111, 63), (127, 15), (128, 5), (129, 1), (160, 48),
+         (223, 2), (224, 0), (225, 1), (240, 16), (255, 3), (256, 0), (257, 31), (300, 4), (449, 2)]
+
+
+@pytest.mark.parametrize("p", ["D", "S"])
+@pytest.mark.parametrize("side", ["L", "R"])
+@pytest.mark.parametrize("n,nrhs", CASES)
+def test_panels(h, p, side, n, nrhs):
+    dt, eps = (np.float64, kt.EPS64) if p == "D" else (np.float32, kt.EPS32)
+    batch, pad = 5, n % 3
+    A = po.gen_spd_shift_batch(60 + n, n, batch).astype(dt).astype(np.float64)
+    bad = 3
+    A[bad][n - 2, n - 2] = -1.0
+    rows, cols = (n, nrhs) if side == "L" else (nrhs, n)
+    lda, ldb = n + pad, max(rows, 1) + pad
+    Ah = np.full((batch, n, lda), np.nan)
+    for c in range(n):
+        Ah[:, c, c:n] = A[:, c, c:]
+    dA = kt.to_dev(Ah, dt)
+    info = kt.to_dev(np.full(batch, -7, np.int32))
+    if nrhs:
+        B = po.gen_rhs_batch(70 + nrhs, rows, cols, batch).astype(dt).astype(np.float64)
+        Bh = np.full((batch, cols, ldb), np.nan)
+        Bh[:, :, :rows] = B
+        dB = kt.to_dev(Bh, dt)
+    f = getattr(h.lib, "kblas%s%s_batch%s" % (p, "posv" if nrhs else "potrf", "" if n % 2 else "_strided"))
+    if n % 2:
+        pA = kt.ptr_array(dA, batch, n * lda)
+        a = (kt.P(pA), lda)
+        if nrhs:
+            pB = kt.ptr_array(dB, batch, cols * ldb)
+            b = (kt.P(pB), ldb)
+    else:
+        a = (kt.P(dA), lda, n * lda)
+        if nrhs:
+            b = (kt.P(dB), ldb, cols * ldb)
+    if nrhs:
+        st = f(h.h, side.encode(), b"L", rows, cols, *a, *b, batch, kt.P(info))
+    else:
+        st = f(h.h, b"L", n, *a, batch, kt.P(info))
+    assert st == pykblas.KBLAS_Success
+    Lh, inf = kt.to_host(dA), kt.to_host(info)
+    for i in range(batch):
+        Ai = po.col(A, i)
+        low = np.tril_indices(n)
+        got = Lh[i, :, :n].T.astype(np.float64)
+        assert np.all(np.isnan(got[np.triu_indices(n, 1)])), i
+        assert np.all(np.isnan(Lh[i, :, n:])), i
+        if i == bad:
+            assert inf[i] == n - 1
+            continue
+        assert inf[i] == 0, i
+        L = np.zeros((n, n))
+        L[low] = got[low]
+        assert np.linalg.norm(L @ L.T - Ai) <= 4 * n * eps * np.linalg.norm(Ai), i
+        if nrhs:
+            Xh = kt.to_host(dB)[i]
+            X, Bi = Xh[:, :rows].T.astype(np.float64), po.col(B, i)
+            assert np.all(np.isnan(Xh[:, rows:])), i
+            _, Xo, _ = po.posv(side, Ai, Bi)
+            assert np.max(np.abs(X - Xo)) <= 64 * n * eps * max(np.max(np.abs(Xo)), 1), i
+            assert po.solve_berr(side, Ai, X, Bi) <= 4 * n * eps, i
