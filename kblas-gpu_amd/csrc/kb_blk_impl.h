@@ -523,60 +523,73 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
 }
 
 // Wave 0's part of a panel: the diagonal block (k0, kb) updated with the k0
-// finished columns, factored, written to memory and to LDS with the inverses
-// of its two 16 x 16 diagonal tiles.  S.flag: 0 or k0 + the failing
-// column (1-based).
+// finished columns, factored and written to memory, its tile (1, 0) and the
+// inverses of its two diagonal tiles to LDS.  S.flag: 0 or k0 + the failing
+// column (1-based).  This is the serial part the other waves wait for, so its
+// products run three to a pair of loads with the next 16 columns' loads in
+// flight (with four loads to three products and none in flight, the update
+// took 28,000 instead of 10,000 cycles a panel at n = 200 in FP32, and SPOTRF
+// n = 200 x 4,000 0.57 instead of 0.40 ms).
 template <typename T>
 KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
 {
+    typedef typename TileV<T>::v4 v4;
     constexpr int LD = KB_BLK_NBK + 1;
     asm volatile("" : "+v"(lane));
     asm volatile("" : "+s"(k0));
     const int i = lane & 15, g = lane >> 4;
-    const int ci = (sizeof(T) == 8) ? 4 * (i & 3) + (i >> 2) : i;   // as in tile_potrf
     T* D = A + k0 + (long)k0 * lda;
-    const T* Lp = A + k0;
-    typename TileV<T>::v4 td[3];
+    // tiles (0,0), (1,0), (1,1) in ll_update's layout: lane (i, g) register r is
+    // row i, column blk_drow(r, g)
+    v4 c[3];
 #pragma unroll
     for (int I = 0; I < 2; ++I)
 #pragma unroll
         for (int J = 0; J <= I; ++J)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = 16 * I + i, col = 16 * J + 4 * g + r;
-                td[tix(I, J)][r] = gld(D + ((row < kb && col <= row) ? row + (long)col * lda : 0));
+                const int row = 16 * I + i, col = 16 * J + blk_drow<T>(r, g);
+                c[tix(I, J)][r] = gld(D + ((row < kb && col <= row) ? row + (long)col * lda : 0));
             }
-    const T *pa[2], *pb[2];
+    const T* p[2];
 #pragma unroll
-    for (int I = 0; I < 2; ++I) {
-        pa[I] = Lp + min(16 * I + ci, kb - 1) + (long)g * lda;
-        pb[I] = Lp + min(16 * I + i, kb - 1) + (long)g * lda;
-    }
-    for (int kc = 0; kc < k0; kc += KB_LL_KC) {   // as in ll_update
-        typename TileV<T>::v4 acc[3];
+    for (int I = 0; I < 2; ++I) p[I] = A + k0 + min(16 * I + i, kb - 1) + (long)g * lda;
+    if (k0 > 0) {
+        constexpr int CH = 16, ST = CH / 4;
+        T x[ST][2], xn[ST][2];
+        auto fetch = [&](T (&y)[ST][2]) {
 #pragma unroll
-        for (int x = 0; x < 3; ++x) acc[x] = typename TileV<T>::v4{T(0), T(0), T(0), T(0)};
-        const int ke = min(kc + KB_LL_KC, k0);
-        for (int k = kc; k < ke; k += 16) {
-            T a[4][2], b[4][2];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < ST; ++u)
 #pragma unroll
                 for (int I = 0; I < 2; ++I) {
-                    a[u][I] = gld(pa[I]);
-                    b[u][I] = gld(pb[I]);
-                    pa[I] += 4 * (long)lda;
-                    pb[I] += 4 * (long)lda;
+                    y[u][I] = gld(p[I]);
+                    p[I] += 4 * (long)lda;
                 }
+        };
+        v4 acc[3];
+        auto mult = [&](const T (&y)[ST][2]) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                acc[0] = mfma16x16x4(a[u][0], b[u][0], acc[0]);
-                acc[1] = mfma16x16x4(a[u][0], b[u][1], acc[1]);
-                acc[2] = mfma16x16x4(a[u][1], b[u][1], acc[2]);
+            for (int u = 0; u < ST; ++u) {
+                acc[0] = mfma16x16x4(y[u][0], y[u][0], acc[0]);
+                acc[1] = mfma16x16x4(y[u][0], y[u][1], acc[1]);
+                acc[2] = mfma16x16x4(y[u][1], y[u][1], acc[2]);
             }
-        }
+        };
+        fetch(x);
+        for (int kc = 0; kc < k0; kc += KB_LL_KC) {   // sums of KB_LL_KC columns, as in ll_update
+            acc[0] = acc[1] = acc[2] = v4{T(0), T(0), T(0), T(0)};
+            const int ke = min(kc + KB_LL_KC, k0);
+            for (int k = kc; k < ke; k += 2 * CH) {   // k0 is a multiple of 32
+                fetch(xn);
+                mult(x);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k + 2 * CH < k0) fetch(x);
+                mult(xn);
+                __builtin_amdgcn_sched_barrier(0);
+            }
 #pragma unroll
-        for (int x = 0; x < 3; ++x) td[x] -= acc[x];
+            for (int q = 0; q < 3; ++q) c[q] -= acc[q];
+        }
     }
     // rows and columns at or beyond kb, and the upper triangle, read as the identity
 #pragma unroll
@@ -585,11 +598,22 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
         for (int J = 0; J <= I; ++J)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = 16 * I + i, col = 16 * J + 4 * g + r;
-                if (!(row < kb && col <= row)) td[tix(I, J)][r] = (row == col) ? T(1) : T(0);
+                const int row = 16 * I + i, col = 16 * J + blk_drow<T>(r, g);
+                const T v = (row < kb && col <= row) ? c[tix(I, J)][r] : (row == col) ? T(1) : T(0);
+                c[tix(I, J)][r] = v;
+                if (sizeof(T) == 8) S.fD[row * LD + col] = v;
             }
+    if constexpr (sizeof(T) == 8) {   // (the FP32 accumulators are in the factorization's layout)
+        wave_lds_sync();
+#pragma unroll
+        for (int I = 0; I < 2; ++I)
+#pragma unroll
+            for (int J = 0; J <= I; ++J)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c[tix(I, J)][r] = S.fD[(16 * I + i) * LD + 16 * J + 4 * g + r];
+    }
     T invd[2] = {T(1), T(1)};
-    const int inf = tile_potrf<T, 2>(td, invd, kb, S.tpan, lane);
+    const int info = tile_potrf<T, 2>(c, invd, kb, S.tpan, lane);
 #pragma unroll
     for (int I = 0; I < 2; ++I)
 #pragma unroll
@@ -597,14 +621,14 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * I + i, col = 16 * J + 4 * g + r;
-                if (row < kb && col <= row) gst(D + row + (long)col * lda, td[tix(I, J)][r]);
-                S.fD[row * LD + col] = (col <= row) ? td[tix(I, J)][r] : T(0);
+                if (row < kb && col <= row) gst(D + row + (long)col * lda, c[tix(I, J)][r]);
+                S.fD[row * LD + col] = (col <= row) ? c[tix(I, J)][r] : T(0);
             }
     if (g == 0) {
         S.sInv[i] = invd[0];
         S.sInv[16 + i] = invd[1];
     }
-    if (lane == 0) S.flag = inf ? k0 + inf : 0;
+    if (lane == 0) S.flag = info ? k0 + info : 0;
     wave_lds_sync();
     // the inverses of both diagonal tiles: DPP row g takes columns 4g..4g+3 of
     // each, lane i of the row holds their row i

@@ -1,8 +1,8 @@
 """GPU parity tests of the workgroup Cholesky (orders above 64) at the edges of
 its panels, against the oracle (orc_posv): orders at and around multiples of
 the 16-row tiles and 32-column panels, orders whose panels need a second round
-of row tiles (above 32 + 12 * 16 = 224 rows, fewer with right-hand sides), and
-right-hand-side counts at and around 16 (they are further row tiles of every
+of row tiles (FP64 above 32 + 6 * 16 rows, FP32 above 32 + 12 * 16, fewer with
+right-hand sides), and right-hand-side counts at and around 16 (they are further row tiles of every
 panel), both sides, both precisions, strided and pointer-array operands.
 
 Bar: the factor's and the solution's normwise backward errors <= 4 n eps, the
