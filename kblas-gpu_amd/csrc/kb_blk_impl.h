@@ -531,7 +531,7 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
 // took 28,000 instead of 10,000 cycles a panel at n = 200 in FP32, and SPOTRF
 // n = 200 x 4,000 0.57 instead of 0.40 ms).
 template <typename T>
-KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
+KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane, T* W)
 {
     typedef typename TileV<T>::v4 v4;
     constexpr int LD = KB_BLK_NBK + 1;
@@ -648,7 +648,11 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) S.fW[b][i * KB_LL_LD + 4 * g + s] = y[b][s] * S.sInv[16 * b + i];
+        for (int s = 0; s < 4; ++s) {
+            const T v = y[b][s] * S.sInv[16 * b + i];
+            S.fW[b][i * KB_LL_LD + 4 * g + s] = v;
+            if (W && 16 * b < kb) gst(W + 16L * (k0 + 16 * b) + 16 * i + 4 * g + s, v);
+        }
 }
 
 // In-place lower Cholesky of an n x n matrix by the whole workgroup.
@@ -656,10 +660,11 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane)
 // forward sweep L Y = B runs inside the factorization, the right-hand sides
 // being further row tiles of every panel; a factorization that fails at panel k
 // leaves B forward-solved in the rows of the panels before k and as it was in
-// the others.
+// the others.  W, if given, receives the inverses of the factor's 16 x 16
+// diagonal tiles (row-major, identity beyond n).
 template <typename T, int CB = 4>
 KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ldb = 0, int side_left = 0,
-                     int nrhs = 0)
+                     int nrhs = 0, T* W = nullptr)
 {
     constexpr int NBK = KB_BLK_NBK, G = ll_g<T>(), NW = KB_BLK_WG / 64;
     static_assert(G <= 4, "one case per tile count below");
@@ -702,7 +707,7 @@ KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ld
             for (int j = 0; j < G; ++j) t[j] = tile(max(min(q0 + j, rest - 1), 0));
             int f;
             if (diag && wave == 0) {
-                ll_diag<T>(A, lda, k0, kb, S, lane);
+                ll_diag<T>(A, lda, k0, kb, S, lane, W);
                 f = ll_group<T, 0>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else if (G >= 4 && cnt == 4) {
                 f = ll_group<T, G >= 4 ? 4 : 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);

@@ -99,6 +99,18 @@ KB_DEV T gld(const T* p)
     return *(const __attribute__((address_space(1))) T*)p;
 }
 
+// A value that is the same in every lane of the wave, as a scalar: sizes and
+// addresses read from memory that the kernel also writes arrive in vector
+// registers otherwise, and everything formed from them stays there.
+KB_DEV int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <typename T>
+KB_DEV T* uniform(T* p)
+{
+    const unsigned long long a = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a), hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    return (T*)(((unsigned long long)hi << 32) | lo);
+}
+
 // gld for one of a group of loads meant to be in flight together: the caller
 // clamps p to a valid address where the value goes unused and selects after
 // the load; the address is kept opaque to the optimizer, which would

@@ -153,40 +153,41 @@ k_vchol_blk(const int* vm, const int* vn, int side_left, BatchArg<T> A, BatchArg
     for (;;) {
         if (threadIdx.x == 0) s_ticket = atomicAdd(q.counter, 1);
         __syncthreads();
-        const int ticket = s_ticket;
+        // scalar, so the sizes and addresses of the matrix stay out of the vector registers
+        const int ticket = uniform(s_ticket);
         __syncthreads();
         if (ticket >= nbig) return;
-        const long mat = q.order[ticket];
-        const int n = vq_order(vm, vn, side_left, mat);
-        const int nrhs = vq_nrhs(vm, vn, side_left, mat);
+        const long mat = uniform(q.order[ticket]);
+        const int n = uniform(vq_order(vm, vn, side_left, mat));
+        const int nrhs = uniform(vq_nrhs(vm, vn, side_left, mat));
         if constexpr (MODE == KB_MODE_SPOSV) {
             // Orders above the register range are solved in FP64 directly
             // (LAPACK dsposv's ITER = -1: full precision for implementation
             // reasons); A receives L as in the dsposv fallback.
-            T* Ap = A.get(mat);
-            const int lda = A.ldim(mat);
-            T* Bp = B.get(mat);
-            T* Xp = X.get(mat);
-            const int ldb = B.ldim(mat), ldx = X.ldim(mat);
+            T* Ap = uniform(A.get(mat));
+            const int lda = uniform(A.ldim(mat));
+            T* Bp = uniform(B.get(mat));
+            T* Xp = uniform(X.get(mat));
+            const int ldb = uniform(B.ldim(mat)), ldx = uniform(X.ldim(mat));
             copy_rhs<T>(Bp, ldb, Xp, ldx, side_left, n, nrhs, threadIdx.x, KB_BLK_WG);
             __syncthreads();
             const int inf = blk_potrf<T, CB>(Ap, lda, n, S, Xp, ldx, side_left, nrhs);
             if (threadIdx.x == 0) { if (info) info[mat] = inf; if (iter) iter[mat] = -1; }
             if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Xp, ldx, side_left, nrhs, S);
         } else {
-            T* Ap = A.get(mat);
-            const int lda = A.ldim(mat);
+            T* Ap = uniform(A.get(mat));
+            const int lda = uniform(A.ldim(mat));
             if constexpr (MODE == KB_MODE_POTRF) {
                 const int inf = blk_potrf<T, CB>(Ap, lda, n, S);
                 if (threadIdx.x == 0 && info) info[mat] = inf;
             } else if constexpr (MODE == KB_MODE_POSV) {
-                T* Bp = B.get(mat);
-                const int ldb = B.ldim(mat);
+                T* Bp = uniform(B.get(mat));
+                const int ldb = uniform(B.ldim(mat));
                 const int inf = blk_potrf<T, CB>(Ap, lda, n, S, Bp, ldb, side_left, nrhs);
                 if (threadIdx.x == 0 && info) info[mat] = inf;
                 if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Bp, ldb, side_left, nrhs, S);
             } else {
-                blk_solve<T, CB>(Ap, lda, n, B.get(mat), B.ldim(mat), side_left, nrhs, S);
+                blk_solve<T, CB>(Ap, lda, n, uniform(B.get(mat)), uniform(B.ldim(mat)), side_left, nrhs, S);
             }
         }
         __syncthreads();
@@ -285,25 +286,25 @@ k_vsposv_big(const int* vm, const int* vn, int side_left, BatchArg<double> A, Ba
     for (;;) {
         if (threadIdx.x == 0) s_ticket = atomicAdd(q.counter, 1);
         __syncthreads();
-        const int ticket = s_ticket;
+        // scalar, so the sizes and addresses of the matrix stay out of the vector registers
+        const int ticket = uniform(s_ticket);
         __syncthreads();
         if (ticket >= nbig) return;
-        const long mat = q.order[ticket];
-        const int n = vq_order(vm, vn, side_left, mat);
-        const int nrhs = vq_nrhs(vm, vn, side_left, mat);
-        double* Ap = A.get(mat);
-        const int lda = A.ldim(mat);
-        const double* Bp = B.get(mat);
-        const int ldb = B.ldim(mat);
-        double* Xp = X.get(mat);
-        const int ldx = X.ldim(mat);
+        const long mat = uniform(q.order[ticket]);
+        const int n = uniform(vq_order(vm, vn, side_left, mat));
+        const int nrhs = uniform(vq_nrhs(vm, vn, side_left, mat));
+        double* Ap = uniform(A.get(mat));
+        const int lda = uniform(A.ldim(mat));
+        const double* Bp = uniform(B.get(mat));
+        const int ldb = uniform(B.ldim(mat));
+        double* Xp = uniform(X.get(mat));
+        const int ldx = uniform(X.ldim(mat));
         if (nrhs <= 0) {
             // nothing to solve (dsposv's quick return)
             if (threadIdx.x == 0) { if (info) info[mat] = 0; if (iter) iter[mat] = 0; }
         } else if (slots && n <= max_n && nrhs <= max_nrhs && n <= KB_SB_MAX_N && nrhs <= KB_SB_MAX_RHS) {
-            float* A32 = slots + (long)blockIdx.x * slot_floats;
-            float* Z = A32 + (long)max_n * max_n;
-            sb_sposv_one(mat, n, nrhs, side_left, Ap, lda, Bp, ldb, Xp, ldx, A32, Z, info, iter, S);
+            sb_sposv_one(mat, n, nrhs, side_left, Ap, lda, Bp, ldb, Xp, ldx, slots + (long)blockIdx.x * slot_floats, info,
+                         iter, S);
         } else {
             // dsposv's full-precision path (ITER = -1); A receives L
             copy_rhs<double>(Bp, ldb, Xp, ldx, side_left, n, nrhs, threadIdx.x, KB_BLK_WG);

@@ -2,13 +2,8 @@
 #include "kb_vchol_impl.h"
 
 // FP32 workspace slot of a workgroup of the mixed phase for orders above the
-// register range: the factor (max_order^2 floats) and the right-hand sides
-// (max_order * max_nrhs floats), rounded up to 256 bytes.
-static long vsposv_slot_floats(int max_order, int max_nrhs)
-{
-    const long f = (long)max_order * max_order + (long)max_order * max_nrhs;
-    return (f + 63) & ~63L;
-}
+// register range (kb_sposv_big.h).
+static long vsposv_slot_floats(int max_order, int max_nrhs) { return sb_slot_floats(max_order, max_nrhs); }
 
 static size_t vsposv_queue_bytes(int batch) { return (kb_vchol_ws_bytes(batch) + 255) & ~(size_t)255; }
 

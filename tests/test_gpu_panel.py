@@ -89,3 +89,59 @@ def test_panels(h, p, side, n, nrhs):
             _, Xo, _ = po.posv(side, Ai, Bi)
             assert np.max(np.abs(X - Xo)) <= 64 * n * eps * max(np.max(np.abs(Xo)), 1), i
             assert po.solve_berr(side, Ai, X, Bi) <= 4 * n * eps, i
+
+
+MIXED_NS = [65, 79, 80, 81, 95, 96, 97, 112, 113, 127, 128, 129, 144, 191, 193, 257, 320, 511]
+
+
+@pytest.mark.parametrize("side", ["L", "R"])
+@pytest.mark.parametrize("nrhs", [1, 15, 16, 17, 33, 48, 64])
+def test_mixed_nonuniform_edges(h, side, nrhs):
+    """the workgroup routine of the non-uniform mixed POSV at the edges of its
+    16-row tiles, 64-row sweep blocks and 16-column right-hand-side blocks:
+    backward error <= 1e-13, refinement within 2 steps of the oracle's dsposv, A
+    and everything outside the solutions left as they were (A's strict upper
+    triangle and the padding hold NaN)"""
+    torch = kt.torch_dev()
+    pad = 3
+    As, Bs, dA, dB, dX, lda, ldb = [], [], [], [], [], [], []
+    for i, n in enumerate(MIXED_NS):
+        A, _ = po.gen_spd_cond(900 + nrhs, i, n, 2.0, 4.0)
+        rows, cols = (n, nrhs) if side == "L" else (nrhs, n)
+        B = po.gen_rhs(901, i, rows, cols)
+        Ah = np.full((n, n + pad), np.nan)
+        for c in range(n):
+            Ah[c, c:n] = A[c:, c]
+        Bh = np.full((cols, rows + pad), np.nan)
+        Bh[:, :rows] = B.T
+        As.append(A)
+        Bs.append(B)
+        dA.append(kt.to_dev(Ah))
+        dB.append(kt.to_dev(Bh))
+        dX.append(torch.full_like(dB[-1], float("nan")))
+        lda.append(n + pad)
+        ldb.append(rows + pad)
+    batch = len(MIXED_NS)
+    dn, dr = kt.to_dev(np.array(MIXED_NS, np.int32)), kt.to_dev(np.full(batch, nrhs, np.int32))
+    m, n = (dn, dr) if side == "L" else (dr, dn)
+    mx = (max(MIXED_NS), nrhs) if side == "L" else (nrhs, max(MIXED_NS))
+    dl, db = kt.to_dev(np.array(lda, np.int32)), kt.to_dev(np.array(ldb, np.int32))
+    ptr = lambda ts: torch.tensor([t.data_ptr() for t in ts], dtype=torch.int64, device="cuda")  # noqa: E731
+    pA, pB, pX = ptr(dA), ptr(dB), ptr(dX)
+    info, it = kt.to_dev(np.full(batch, -7, np.int32)), kt.to_dev(np.full(batch, -99, np.int32))
+    h.lib.kblas_sposv_vbatch_wsquery(h.h, nrhs, max(MIXED_NS), batch)
+    assert h.lib.kblasAllocateWorkspace(h.h) == pykblas.KBLAS_Success
+    st = h.lib.kblasDsposv_vbatch(h.h, side.encode(), b"L", kt.P(m), kt.P(n), mx[0], mx[1], kt.P(pA), kt.P(dl),
+                                  kt.P(pB), kt.P(db), kt.P(pX), kt.P(db), batch, kt.P(info), kt.P(it))
+    assert st == pykblas.KBLAS_Success
+    inf, itr = kt.to_host(info), kt.to_host(it)
+    for i, n in enumerate(MIXED_NS):
+        assert inf[i] == 0 and itr[i] >= 0, (n, inf[i], itr[i])
+        Ah, Xh = kt.to_host(dA[i]), kt.to_host(dX[i])
+        assert np.array_equal(np.tril(Ah[:, :n].T), np.tril(As[i])), n
+        rows = Bs[i].shape[0]
+        assert np.all(np.isnan(Xh[:, rows:])), n
+        assert po.solve_berr(side, As[i], Xh[:, :rows].T, Bs[i]) <= 1e-13, n
+        if n <= 129:
+            _, _, want = po.sposv(side, As[i], Bs[i])
+            assert abs(int(itr[i]) - want) <= 2, (n, itr[i], want)
