@@ -91,7 +91,7 @@ KB_DEV kb_d2 gld2u(const double* p)
 
 // A32 := FP32 copy of the lower triangle of A (ld n), SB_U columns at a time;
 // big is set when an entry exceeds FP32 range.
-constexpr int SB_U = 8;
+constexpr int SB_U = 16;
 
 KB_DEV void sb_convert(const double* A, int lda, int n, float* A32, bool& big)
 {
