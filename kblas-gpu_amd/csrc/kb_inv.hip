@@ -7,7 +7,8 @@
 //   TRMM   B := alpha op(L) B  or  alpha B op(L)
 //                                    src/batch_triangular/Xtrmm_batch_kernels.cuh:37-175
 //
-// Orders up to 64: k_inv_reg, 64 / NL matrices per wave, registers (below).
+// POTRI up to 32 (real): k_potri_dpp, four matrices per wave, no LDS (below).
+// Otherwise orders up to 64: k_inv_reg, 64 / NL matrices per wave, registers.
 // Larger orders: k_inv, one workgroup per matrix, one thread per row (TRTRI)
 // or column (LAUUM) of the matrix, so n <= KB_INV_MAX_N.  The matrix is staged in LDS when its
 // n x n block fits in KB_INV_LDS bytes and is worked on in place in HBM
@@ -237,6 +238,89 @@ k_inv_reg(int op, int unit, int n, BatchArg<T> A, int* info, const int* skip, in
     if (live && info && r == 0) info[b] = inf;
 }
 
+// ------------------------------------- POTRI, n <= 32: four matrices a wave ----
+// A matrix sits in one 16-lane DPP row, lane i with rows i and (NB = 32) 16 + i
+// of the padded triangle in registers.  Lane a then forms row a of U = L^-T by
+// substitution, u_j = x_j / L(j,j), x_k -= u_j L(k,j) for k > j, where L(k,j) is
+// lane k's register j read through DPP inside the FMA; and row a of the result,
+// sum_k U(a,k) U(c,k) over k ascending, with U(c,k) from lane c the same way.  No
+// LDS: the register form above is bound by its LDS broadcasts (every lane reads
+// the whole triangle twice).  POTRI n = 32 x 10,000 FP64: 65 -> 34 us,
+// POTI with the factorization before it 82 -> 51 us; n = 16 x 20,000 24 -> 13 us.
+template <int NB, typename T>
+__global__ void __launch_bounds__(64)
+k_potri_dpp(int n, BatchArg<T> A, int* info, const int* skip, int batch)
+{
+    constexpr int NS = NB / 16;
+    const int lane = threadIdx.x, i = lane & 15;
+    const long b = (long)blockIdx.x * 4 + (lane >> 4);
+    const long bv = b < batch ? b : batch - 1;
+    const bool live = b < batch && !(skip && skip[bv] != 0);
+    T* G = A.get(bv);
+    const int lda = A.ldim(bv);
+    T l[NS][NB];   // slot s: row 16 s + i, columns 0 .. 16 s + 15 (identity beyond n)
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int k = 0; k < 16 * (s + 1); ++k) {
+            const int r = 16 * s + i;
+            const bool in = r < n && k <= r;
+            const T v = gld_opaque(G + (in ? r + (long)k * lda : 0));
+            l[s][k] = in ? v : (r == k) ? T(1) : T(0);
+        }
+    T iv[NS];
+    int inf = 0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        T d = T(1);
+#pragma unroll
+        for (int k = 16 * s; k < 16 * (s + 1); ++k) d = (16 * s + i == k) ? l[s][k] : d;
+        // first exactly zero diagonal element of this lane's matrix
+        const unsigned zm = (unsigned)(__ballot(d == T(0)) >> (lane & 48)) & 0xffffu;
+        if (inf == 0 && zm) inf = 16 * s + __builtin_ctz(zm) + 1;
+        iv[s] = kb_rcp<T>(d);
+    }
+    // U: slot s has x[s][k] for k >= 16 s (zero before the row's own column)
+    T x[NS][NB];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+        for (int k = 16 * s; k < NB; ++k) x[s][k] = (16 * s + i == k) ? T(1) : T(0);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const T ij = row_bcast<T>(iv[j >> 4], j);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            if (j >= 16 * s) {
+                x[s][j] *= ij;
+#pragma unroll
+                for (int k = j + 1; k < NB; ++k) fnmac_rowk<T>(x[s][k], l[k >> 4][j], x[s][j], k);
+            }
+        }
+    }
+    // rows of the result, a column at a time
+    const bool wr = live && inf == 0;
+    T* q = G + i;
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+        T o[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            o[s] = T(0);
+            if (c >= 16 * (s + 1)) continue;   // above the diagonal
+            const int t = c >> 4;              // column c is row c - 16 t of slot t
+#pragma unroll
+            for (int k = (c > 16 * s) ? c : 16 * s; k < NB; ++k) fmac_rowk<T>(o[s], x[t][k], x[s][k], c);
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+            if (wr && c <= 16 * s + i && 16 * s + i < n && c < n) gst(q + 16 * s, o[s]);
+        q += lda;
+        asm volatile("" : "+v"(q));
+    }
+    if (live && info && i == 0) info[b] = inf <= n ? inf : 0;
+}
+
 // ---------------------------------------------------------------- TRMM ----
 // Element (r, c) of alpha op(L) B (left, L of order m) or alpha B op(L)
 // (right, L of order n), read from the panel copy P (ldp rows) of B.
@@ -365,6 +449,14 @@ static int launch_inv(int op, int unit, int n, kb_mat_t A, int* info, const int*
     // register form: real types up to 64, single complex up to 16 (above, its
     // rows would not fit in registers), double complex never
     constexpr int REG_MAX = __is_same(T, kb_cd) ? 0 : __is_same(T, kb_cf) ? 16 : 64;
+    if constexpr (REG_MAX >= 64) {
+        if (op == KB_INV_OP_POTRI && n <= 32) {
+            const dim3 grid((batch + 3) / 4);
+            if (n <= 16) hipLaunchKernelGGL((k_potri_dpp<16, T>), grid, dim3(64), 0, s, n, to_arg<T>(A), info, skip, batch);
+            else hipLaunchKernelGGL((k_potri_dpp<32, T>), grid, dim3(64), 0, s, n, to_arg<T>(A), info, skip, batch);
+            return (int)hipGetLastError();
+        }
+    }
     if constexpr (REG_MAX >= 16) {
         if (n <= 16) {
             hipLaunchKernelGGL((k_inv_reg<T, 16>), dim3((batch + 3) / 4), dim3(64), 0, s, op, unit, n, to_arg<T>(A),
