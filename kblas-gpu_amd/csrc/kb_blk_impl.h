@@ -35,7 +35,6 @@
 
 constexpr int KB_BLK_NBK = 32;
 constexpr int KB_BLK_WG = 256;
-constexpr int KB_BLK_RC = 64;   // right-hand sides per pass of the solve
 constexpr int KB_LL_LD = 17;    // pitch of a staged 16 x 16 tile
 // 16-row tiles a wave holds at once (C and the running sums: FP64 16 VGPRs each
 // per tile).  FP64: 2 fill the 128 VGPRs that four workgroups per CU leave; 3
@@ -46,11 +45,12 @@ template <> constexpr int ll_g<double>() { return 2; }
 template <> constexpr int ll_g<float>() { return 4; }
 
 // The factorization's blocks and the solve's staging are never live together.
-template <typename T>
+// CB: the widest pass of the solve, in blocks of 16 right-hand sides.
+template <typename T, int CB = 4>
 struct BlkSmem {
     union {
         struct {
-            T sY[KB_BLK_RC * (KB_BLK_NBK + 1)];   // the solve's staging of a block of the solution
+            T sY[16 * CB * (KB_BLK_NBK + 1)];     // the solve's staging of a block of the solution
             T sD[KB_BLK_NBK * (KB_BLK_NBK + 1)];  // the diagonal block
         };
         struct {
@@ -74,17 +74,17 @@ KB_DEV T& rhs_at(T* B, int ldb, int side_left, int i, int c)
 // can issue the loads of the next block before working on the current one:
 // blk_diag_fetch reads this thread's elements (e = tid + 256 m) into
 // registers, blk_diag_put writes them to LDS with the inverse diagonal.
-constexpr int KB_BLK_DPT = KB_BLK_NBK * KB_BLK_NBK / KB_BLK_WG;   // elements per thread
+template <int W> constexpr int blk_dpt() { return KB_BLK_NBK * KB_BLK_NBK / W; }   // elements per thread of W
 
-template <typename T>
-KB_DEV void blk_diag_fetch(T (&v)[KB_BLK_DPT], const T* L, int lda, int k0, int kb)
+template <typename T, int W>
+KB_DEV void blk_diag_fetch(T (&v)[blk_dpt<W>()], const T* L, int lda, int k0, int kb)
 {
     constexpr int NBK = KB_BLK_NBK;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));   // lane-dependent values formed per call, not kept live across
 #pragma unroll
-    for (int m = 0; m < KB_BLK_DPT; ++m) {
-        const int e = tid + KB_BLK_WG * m;
+    for (int m = 0; m < blk_dpt<W>(); ++m) {
+        const int e = tid + W * m;
         const int r = e % NBK, c = e / NBK;
         const bool in = r < kb && c <= r;
         const T x = gld(L + (in ? (k0 + r) + (long)(k0 + c) * lda : 0));
@@ -92,15 +92,15 @@ KB_DEV void blk_diag_fetch(T (&v)[KB_BLK_DPT], const T* L, int lda, int k0, int 
     }
 }
 
-template <typename T>
-KB_DEV void blk_diag_put(const T (&v)[KB_BLK_DPT], int kb, BlkSmem<T>& S, int unit = 0)
+template <typename T, int CB, int W>
+KB_DEV void blk_diag_put(const T (&v)[blk_dpt<W>()], int kb, BlkSmem<T, CB>& S, int unit = 0)
 {
     constexpr int NBK = KB_BLK_NBK;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
 #pragma unroll
-    for (int m = 0; m < KB_BLK_DPT; ++m) {
-        const int e = tid + KB_BLK_WG * m;
+    for (int m = 0; m < blk_dpt<W>(); ++m) {
+        const int e = tid + W * m;
         const int r = e % NBK, c = e / NBK;
         S.sD[r * (NBK + 1) + c] = v[m];
         if (r == c) S.sInv[r] = (r < kb && !unit) ? T(1) / v[m] : T(1);
@@ -118,14 +118,14 @@ KB_DEV int blk_drow(int q, int g)
 }
 
 // Substitution with the staged diagonal block (sD, sInv) for the NS groups of
-// 16 right-hand sides of a pass: DPP row (wave, lg) of the workgroup takes
-// right-hand sides c = 16 s + 4 wave + lg, lane li of the row holds block rows
+// W / 16 right-hand sides of a pass: DPP row (wave, lg) of the workgroup takes
+// right-hand sides c = W / 16 s + 4 wave + lg, lane li of the row holds block rows
 // li and 16 + li, and y(j) comes from lane j by DPP; the NS independent
 // substitutions are interleaved and share the LDS reads of L.
 // FWD: L_D y = b, else L_D^T x = y; the result also goes to sY (right-hand
 // side major) for the off-diagonal update that follows.  b is read as sc * b.
-template <typename T, int NS, bool FWD>
-KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T>& S, T* sY,
+template <typename T, int NS, bool FWD, int CB, int W>
+KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T, CB>& S, T* sY,
                            T sc = T(1))
 {
     constexpr int NBK = KB_BLK_NBK;
@@ -141,7 +141,7 @@ KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0,
     for (int h = 0; h < 2; ++h) iv[h] = S.sInv[16 * h + li];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int c = 16 * s + 4 * wave + lg;
+        const int c = W / 16 * s + 4 * wave + lg;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int r = 16 * h + li;
@@ -172,7 +172,7 @@ KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0,
     }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        const int c = 16 * s + 4 * wave + lg;
+        const int c = W / 16 * s + 4 * wave + lg;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int r = 16 * h + li;
@@ -185,19 +185,22 @@ KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0,
     }
 }
 
-// ns groups of 16 right-hand sides, ns <= CB (the widest pass instantiated)
-template <typename T, bool FWD, int CB>
-KB_DEV void blk_diag_subst_n(int ns, T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T>& S,
-                             T* sY, T sc = T(1))
+// all rc right-hand sides of a pass of up to 16 CB
+template <typename T, bool FWD, int CB, int W>
+KB_DEV void blk_diag_subst_n(T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T, CB>& S, T* sY,
+                             T sc = T(1))
 {
-    if (CB == 2 || ns <= 2) {
-        if (ns == 1) blk_diag_subst<T, 1, FWD>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
-        else blk_diag_subst<T, 2, FWD>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+    constexpr int MX = 16 * CB / (W / 16);   // groups of a full pass
+    static_assert(MX == 2 || MX == 4, "one case per group count");
+    const int ns = (rc + W / 16 - 1) / (W / 16);
+    if (MX == 2 || ns <= 2) {
+        if (ns == 1) blk_diag_subst<T, 1, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+        else blk_diag_subst<T, 2, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
         return;
     }
-    if constexpr (CB > 2) {
-        if (ns == 3) blk_diag_subst<T, 3, FWD>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
-        else blk_diag_subst<T, 4, FWD>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+    if constexpr (MX > 2) {
+        if (ns == 3) blk_diag_subst<T, 3, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+        else blk_diag_subst<T, 4, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
     }
 }
 
@@ -208,7 +211,7 @@ KB_DEV void blk_diag_subst_n(int ns, T* B, int ldb, int side_left, int k0, int k
 // staged in sY (right-hand side major).  Each wave takes 16-row blocks: the
 // L fragment (eight K steps of 4) and the B blocks of the NCB column blocks of
 // 16 right-hand sides are loaded together, then NCB independent MFMA chains.
-template <typename T, bool TRANS, int NCB>
+template <typename T, bool TRANS, int NCB, int W>
 KB_DEV void blk_update_rows(const T* L, int lda, T* B, int ldb, int side_left, int k0, int kb, int r_lo,
                             int r_hi, int c0, int rc, const T* sY, T sc = T(1))
 {
@@ -217,7 +220,7 @@ KB_DEV void blk_update_rows(const T* L, int lda, T* B, int ldb, int side_left, i
     asm volatile("" : "+v"(tid));   // lane-dependent offsets stay local (as in blk_diag_subst)
     const int wave = tid >> 6, lane = tid & 63;
     const int li = lane & 15, lg = lane >> 4;
-    for (int r0 = r_lo + 16 * wave; r0 < r_hi; r0 += KB_BLK_WG / 4) {
+    for (int r0 = r_lo + 16 * wave; r0 < r_hi; r0 += W / 4) {
         T a[NBK / 4];
 #pragma unroll
         for (int q = 0; q < NBK / 4; ++q) {
@@ -265,18 +268,18 @@ KB_DEV void blk_update_rows(const T* L, int lda, T* B, int ldb, int side_left, i
     }
 }
 
-template <typename T, bool TRANS, int CB>
+template <typename T, bool TRANS, int CB, int W>
 KB_DEV void blk_update_rows_n(int ncb, const T* L, int lda, T* B, int ldb, int side_left, int k0, int kb, int r_lo,
                               int r_hi, int c0, int rc, const T* sY, T sc = T(1))
 {
     if (CB == 2 || ncb <= 2) {
-        if (ncb == 1) blk_update_rows<T, TRANS, 1>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
-        else blk_update_rows<T, TRANS, 2>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
+        if (ncb == 1) blk_update_rows<T, TRANS, 1, W>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
+        else blk_update_rows<T, TRANS, 2, W>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
         return;
     }
     if constexpr (CB > 2) {
-        if (ncb == 3) blk_update_rows<T, TRANS, 3>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
-        else blk_update_rows<T, TRANS, 4>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
+        if (ncb == 3) blk_update_rows<T, TRANS, 3, W>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
+        else blk_update_rows<T, TRANS, 4, W>(L, lda, B, ldb, side_left, k0, kb, r_lo, r_hi, c0, rc, sY, sc);
     }
 }
 
@@ -285,19 +288,18 @@ KB_DEV void blk_update_rows_n(int ncb, const T* L, int lda, T* B, int ldb, int s
 // block column of L (all right-hand sides, in passes of up to 16 CB: a
 // narrower pass needs fewer registers, a wider one streams L fewer times).
 // sc scales the right-hand sides as they are first read (the first step).
-template <typename T, int CB = 4>
+template <typename T, int CB, int W>
 KB_DEV void blk_fwd_step(const T* L, int lda, int n, int k0, int kb, T* B, int ldb, int side_left, int nrhs,
-                         BlkSmem<T>& S, T sc = T(1))
+                         BlkSmem<T, CB>& S, T sc = T(1))
 {
     constexpr int RC = 16 * CB;
-    static_assert(RC <= KB_BLK_RC, "the staging holds KB_BLK_RC right-hand sides");
     T* sY = S.sY;   // RC x (NBK + 1) staging of the block's solution
     for (int c0 = 0; c0 < nrhs; c0 += RC) {
         const int rc = min(RC, nrhs - c0);
         const int ncb = (rc + 15) / 16;
-        blk_diag_subst_n<T, true, CB>(ncb, B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+        blk_diag_subst_n<T, true, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
         __syncthreads();
-        blk_update_rows_n<T, false, CB>(ncb, L, lda, B, ldb, side_left, k0, kb, k0 + kb, n, c0, rc, sY, sc);
+        blk_update_rows_n<T, false, CB, W>(ncb, L, lda, B, ldb, side_left, k0, kb, k0 + kb, n, c0, rc, sY, sc);
         __syncthreads();
     }
 }
@@ -305,55 +307,55 @@ KB_DEV void blk_fwd_step(const T* L, int lda, int n, int k0, int kb, T* B, int l
 // Forward sweep L Y = alpha B over 32-row blocks (right-looking), the next
 // diagonal block fetched while the current one is used; unit: the diagonal
 // of L is taken as 1 (not read).
-template <typename T, int CB = 4>
-KB_DEV void blk_solve_fwd(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T>& S,
+template <typename T, int CB = 4, int W = KB_BLK_WG>
+KB_DEV void blk_solve_fwd(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T, CB>& S,
                           T alpha = T(1), int unit = 0)
 {
     constexpr int NBK = KB_BLK_NBK;
-    T dnext[KB_BLK_DPT];
-    blk_diag_fetch<T>(dnext, L, lda, 0, min(NBK, n));
+    T dnext[blk_dpt<W>()];
+    blk_diag_fetch<T, W>(dnext, L, lda, 0, min(NBK, n));
     for (int k0 = 0; k0 < n; k0 += NBK) {
         const int kb = min(NBK, n - k0);
-        blk_diag_put<T>(dnext, kb, S, unit);
-        if (k0 + NBK < n) blk_diag_fetch<T>(dnext, L, lda, k0 + NBK, min(NBK, n - k0 - NBK));
-        blk_fwd_step<T, CB>(L, lda, n, k0, kb, B, ldb, side_left, nrhs, S, k0 == 0 ? alpha : T(1));
+        blk_diag_put<T, CB, W>(dnext, kb, S, unit);
+        if (k0 + NBK < n) blk_diag_fetch<T, W>(dnext, L, lda, k0 + NBK, min(NBK, n - k0 - NBK));
+        blk_fwd_step<T, CB, W>(L, lda, n, k0, kb, B, ldb, side_left, nrhs, S, k0 == 0 ? alpha : T(1));
     }
 }
 
 // Backward sweep L^T X = alpha Y over 32-row blocks (right-looking: after
 // each block's substitution the rows above it are updated); unit as above.
-template <typename T, int CB = 4>
-KB_DEV void blk_solve_bwd(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T>& S,
+template <typename T, int CB = 4, int W = KB_BLK_WG>
+KB_DEV void blk_solve_bwd(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T, CB>& S,
                           T alpha = T(1), int unit = 0)
 {
     constexpr int NBK = KB_BLK_NBK, RC = 16 * CB;
     T* sY = S.sY;
-    T dnext[KB_BLK_DPT];
+    T dnext[blk_dpt<W>()];
     const int nblk = (n + NBK - 1) / NBK;
-    blk_diag_fetch<T>(dnext, L, lda, (nblk - 1) * NBK, n - (nblk - 1) * NBK);
+    blk_diag_fetch<T, W>(dnext, L, lda, (nblk - 1) * NBK, n - (nblk - 1) * NBK);
     for (int bk = nblk - 1; bk >= 0; --bk) {
         const int k0 = bk * NBK;
         const int kb = min(NBK, n - k0);
-        blk_diag_put<T>(dnext, kb, S, unit);
-        if (bk > 0) blk_diag_fetch<T>(dnext, L, lda, k0 - NBK, NBK);
+        blk_diag_put<T, CB, W>(dnext, kb, S, unit);
+        if (bk > 0) blk_diag_fetch<T, W>(dnext, L, lda, k0 - NBK, NBK);
         const T sc = bk == nblk - 1 ? alpha : T(1);
         for (int c0 = 0; c0 < nrhs; c0 += RC) {
             const int rc = min(RC, nrhs - c0);
             const int ncb = (rc + 15) / 16;
-            blk_diag_subst_n<T, false, CB>(ncb, B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+            blk_diag_subst_n<T, false, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
             __syncthreads();
-            blk_update_rows_n<T, true, CB>(ncb, L, lda, B, ldb, side_left, k0, kb, 0, k0, c0, rc, sY, sc);
+            blk_update_rows_n<T, true, CB, W>(ncb, L, lda, B, ldb, side_left, k0, kb, 0, k0, c0, rc, sY, sc);
             __syncthreads();
         }
     }
 }
 
 // Solve (L L^T) X = B for nrhs vectors stored by rhs_at(); L lower in A.
-template <typename T, int CB = 4>
-KB_DEV void blk_solve(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T>& S)
+template <typename T, int CB = 4, int W = KB_BLK_WG>
+KB_DEV void blk_solve(const T* L, int lda, int n, T* B, int ldb, int side_left, int nrhs, BlkSmem<T, CB>& S)
 {
-    blk_solve_fwd<T, CB>(L, lda, n, B, ldb, side_left, nrhs, S);
-    blk_solve_bwd<T, CB>(L, lda, n, B, ldb, side_left, nrhs, S);
+    blk_solve_fwd<T, CB, W>(L, lda, n, B, ldb, side_left, nrhs, S);
+    blk_solve_bwd<T, CB, W>(L, lda, n, B, ldb, side_left, nrhs, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -471,8 +473,8 @@ KB_DEV typename TileV<T>::v4 ll_apply(const T* W, int li, int lg, const typename
 // X1^T = L11^-1 C1^T, X2^T = L22^-1 (C2^T - L21 X1^T).  A 16 x 16 accumulator is
 // itself the second operand of the next product (register s of lane group g
 // holds row kmap(s, g)), so nothing leaves the registers.
-template <typename T>
-KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const BlkSmem<T>& S,
+template <typename T, int CB>
+KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const BlkSmem<T, CB>& S,
                      typename TileV<T>::v4 (&c)[2])
 {
     constexpr int LD = KB_BLK_NBK + 1;
@@ -498,9 +500,9 @@ KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const B
 // One wave's NT tiles of a panel: update, wait for the diagonal block (first:
 // every wave of the workgroup passes exactly one barrier here, in ll_diag's
 // branch or in one of these), solve.  Returns S.flag.
-template <typename T, int NT>
+template <typename T, int NT, int CB>
 KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTile<T>* t, int li, int lg,
-                    const BlkSmem<T>& S)
+                    const BlkSmem<T, CB>& S)
 {
     typename TileV<T>::v4 c[NT > 0 ? NT : 1][2];
     if constexpr (NT > 0) ll_update<T, NT>(Lp, lda, kb, k0, t, li, lg, c);
@@ -515,7 +517,7 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
         asm volatile("" : "+s"(k0));
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            ll_solve<T>(t[j], kb, k0, li, lg, S, c[j]);
+            ll_solve<T, CB>(t[j], kb, k0, li, lg, S, c[j]);
             __builtin_amdgcn_sched_barrier(0);   // one tile's products at a time (registers)
         }
     }
@@ -530,8 +532,8 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
 // flight (with four loads to three products and none in flight, the update
 // took 28,000 instead of 10,000 cycles a panel at n = 200 in FP32, and SPOTRF
 // n = 200 x 4,000 0.57 instead of 0.40 ms).
-template <typename T>
-KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane, T* W)
+template <typename T, int CB>
+KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, T* W)
 {
     typedef typename TileV<T>::v4 v4;
     constexpr int LD = KB_BLK_NBK + 1;
@@ -660,13 +662,13 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T>& S, int lane, T* W
 // forward sweep L Y = B runs inside the factorization, the right-hand sides
 // being further row tiles of every panel; a factorization that fails at panel k
 // leaves B forward-solved in the rows of the panels before k and as it was in
-// the others.  W, if given, receives the inverses of the factor's 16 x 16
+// the others.  Wt, if given, receives the inverses of the factor's 16 x 16
 // diagonal tiles (row-major, identity beyond n).
-template <typename T, int CB = 4>
-KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ldb = 0, int side_left = 0,
-                     int nrhs = 0, T* W = nullptr)
+template <typename T, int CB = 4, int W = KB_BLK_WG>
+KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T, CB>& S, T* B = nullptr, int ldb = 0, int side_left = 0,
+                     int nrhs = 0, T* Wt = nullptr)
 {
-    constexpr int NBK = KB_BLK_NBK, G = ll_g<T>(), NW = KB_BLK_WG / 64;
+    constexpr int NBK = KB_BLK_NBK, G = ll_g<T>(), NW = W / 64;
     static_assert(G <= 4, "one case per tile count below");
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));   // lane-dependent values formed per call, not kept live across
@@ -707,18 +709,18 @@ KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ld
             for (int j = 0; j < G; ++j) t[j] = tile(max(min(q0 + j, rest - 1), 0));
             int f;
             if (diag && wave == 0) {
-                ll_diag<T>(A, lda, k0, kb, S, lane, W);
-                f = ll_group<T, 0>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                ll_diag<T, CB>(A, lda, k0, kb, S, lane, Wt);
+                f = ll_group<T, 0, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else if (G >= 4 && cnt == 4) {
-                f = ll_group<T, G >= 4 ? 4 : 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                f = ll_group<T, G >= 4 ? 4 : 1, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else if (G >= 3 && cnt == 3) {
-                f = ll_group<T, G >= 3 ? 3 : 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                f = ll_group<T, G >= 3 ? 3 : 1, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else if (cnt == 2) {
-                f = ll_group<T, 2>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                f = ll_group<T, 2, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else if (cnt == 1) {
-                f = ll_group<T, 1>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                f = ll_group<T, 1, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             } else {
-                f = ll_group<T, 0>(diag, A + k0, lda, kb, k0, t, li, lg, S);
+                f = ll_group<T, 0, CB>(diag, A + k0, lda, kb, k0, t, li, lg, S);
             }
             if (f) return f;
             base += round;
@@ -730,26 +732,26 @@ KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T>& S, T* B = nullptr, int ld
 
 // CB = 2: passes of 32 right-hand sides, few enough registers for four
 // waves per SIMD; CB = 4: passes of 64 (L streamed half as often), three.
-template <typename T, int MODE, int CB>
-__global__ void __launch_bounds__(KB_BLK_WG) __attribute__((amdgpu_waves_per_eu(CB == 2 ? 4 : 2)))
+template <typename T, int MODE, int CB, int W>
+__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(CB == 2 ? 4 : 2)))
 k_blk_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* info, int batch)
 {
-    __shared__ BlkSmem<T> S;
+    __shared__ BlkSmem<T, CB> S;
     for (long mat = blockIdx.x; mat < batch; mat += gridDim.x) {
-        T* Ap = A.get(mat);
-        const int lda = A.ldim(mat);
+        T* Ap = uniform(A.get(mat));
+        const int lda = uniform(A.ldim(mat));
         int inf = 0;
         if constexpr (MODE == KB_MODE_POTRF) {
-            inf = blk_potrf<T, CB>(Ap, lda, n, S);
+            inf = blk_potrf<T, CB, W>(Ap, lda, n, S);
             if (threadIdx.x == 0 && info) info[mat] = inf;
         } else if constexpr (MODE == KB_MODE_POSV) {
-            T* Bp = B.get(mat);
-            const int ldb = B.ldim(mat);
-            inf = blk_potrf<T, CB>(Ap, lda, n, S, Bp, ldb, side_left, nrhs);
+            T* Bp = uniform(B.get(mat));
+            const int ldb = uniform(B.ldim(mat));
+            inf = blk_potrf<T, CB, W>(Ap, lda, n, S, Bp, ldb, side_left, nrhs);
             if (threadIdx.x == 0 && info) info[mat] = inf;
-            if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Bp, ldb, side_left, nrhs, S);
+            if (inf == 0) blk_solve_bwd<T, CB, W>(Ap, lda, n, Bp, ldb, side_left, nrhs, S);
         } else {
-            blk_solve<T, CB>(Ap, lda, n, B.get(mat), B.ldim(mat), side_left, nrhs, S);
+            blk_solve<T, CB, W>(Ap, lda, n, uniform(B.get(mat)), uniform(B.ldim(mat)), side_left, nrhs, S);
         }
         __syncthreads();
     }
@@ -757,17 +759,32 @@ k_blk_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* in
 
 // Passes of 32 right-hand sides when the count allows (POTRF: none), else 64.
 constexpr int KB_BLK_NARROW = 32;
+// Two waves per matrix instead of four where a panel has too few row tiles to
+// keep three waves busy while the first factors the diagonal block: twice the
+// matrices per CU then hide its chain.  Only for batches that fill the chip with
+// four waves each (256 CUs x 4 workgroups), and up to the order, or order and
+// right-hand sides, where the four waves' updates win again.  256 -> 128
+// threads (us, with the copies that restore the inputs): DPOTRF n = 80 x 10,000
+// 546 -> 448, n = 200 x 2,000 585 -> 560, n = 256 x 4,096 1,762 -> 1,810; DPOSV n
+// = 100 x 5,000, 8 right-hand sides 611 -> 505, n = 200 x 3,000, 4 right-hand
+// sides 1,088 -> 1,058, 30 right-hand sides 1,340 -> 1,433; DPOTRS n = 224 x
+// 1,100, 16 right-hand sides 192 -> 213.
+constexpr int KB_BLK_FULL = 1024;
 
 template <typename T, int MODE>
 static void launch_blk_mode(int n, int nrhs, int side_left, BatchArg<T> a, BatchArg<T> b, int* info, int batch,
                             int grid, hipStream_t s)
 {
-    if (MODE == KB_MODE_POTRF || nrhs <= KB_BLK_NARROW)
-        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a, b, info,
+    const bool narrow = MODE == KB_MODE_POTRF || nrhs <= KB_BLK_NARROW;
+    if (narrow && batch > KB_BLK_FULL && n <= (MODE == KB_MODE_POTRF || nrhs <= 4 ? 224 : nrhs <= 16 ? 192 : 128))
+        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, 128>), dim3(grid), dim3(128), 0, s, n, nrhs, side_left, a, b, info,
                            batch);
+    else if (narrow)
+        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, KB_BLK_WG>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a,
+                           b, info, batch);
     else
-        hipLaunchKernelGGL((k_blk_chol<T, MODE, 4>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a, b, info,
-                           batch);
+        hipLaunchKernelGGL((k_blk_chol<T, MODE, 4, KB_BLK_WG>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a,
+                           b, info, batch);
 }
 
 // Batched lower TRSM for orders above the register range: one sweep of the
@@ -779,7 +796,7 @@ __global__ void __launch_bounds__(KB_BLK_WG) __attribute__((amdgpu_waves_per_eu(
 k_blk_trsm(int n0, int nrhs0, int side_left, int unit, T alpha, BatchArg<T> A, BatchArg<T> B, int batch,
            const int* vm, const int* vn)
 {
-    __shared__ BlkSmem<T> S;
+    __shared__ BlkSmem<T, CB> S;
     for (long mat = blockIdx.x; mat < batch; mat += gridDim.x) {
         int n = n0, nrhs = nrhs0;
         if (vm) {   // non-uniform: this matrix's order and right-hand-side count

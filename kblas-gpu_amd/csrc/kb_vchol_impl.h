@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(KB_BLK_WG) __attribute__((amdgpu_waves_per_eu(
 k_vchol_blk(const int* vm, const int* vn, int side_left, BatchArg<T> A, BatchArg<T> B, BatchArg<T> X,
             int* info, int* iter, int batch, void* ws)
 {
-    __shared__ BlkSmem<T> S;
+    __shared__ BlkSmem<T, CB> S;
     __shared__ int s_ticket;
     VQueue q = vq_view(ws, batch);
     const int nbig = q.counter[1];
