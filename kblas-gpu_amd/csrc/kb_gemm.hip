@@ -5,8 +5,8 @@
 //   GEMM  C := alpha op(A) op(B) + beta C
 //   SYRK  the lower (or upper) triangle of C := alpha op(A) op(A)^T + beta C
 //
-// GEMM with m, n >= 64: 64 x 64 workgroup tiles through LDS (k_gemm_lds below).
-// Otherwise, and for SYRK: one wavefront per TM x TM output tile (TM = 16 or 32), the tile built from
+// GEMM with m, n >= 64, and SYRK of some orders (gm_dispatch): 64 x 64 workgroup
+// tiles through LDS (k_gemm_lds below).  Otherwise: one wavefront per TM x TM output tile (TM = 16 or 32), the tile built from
 // 16 x 16 x 4 matrix-core products (FP64 or FP32).  The product is formed
 // transposed, D = op(B)^T op(A)^T, so that the accumulator's lanes run down
 // the columns of C and the read-modify-write of C is coalesced.  Operand
@@ -169,7 +169,7 @@ k_gemm_mfma(int m, int n, int k, T alpha, BatchArgO<T> A, BatchArgO<T> B, T beta
 // the current chunk's products run (two LDS buffers, one barrier per chunk).
 // ---------------------------------------------------------------------------
 constexpr int GL_TM = 64, GL_KC = 16, GL_LD = GL_TM + 2;
-// smallest m and n for the workgroup tile (smaller products, and SYRK, keep the wavefront tiles)
+// smallest m and n for the workgroup tile (smaller products keep the wavefront tiles)
 constexpr int GM_LDS_MIN = 64;
 
 template <typename T, bool TA, bool TB>
@@ -245,6 +245,8 @@ k_gemm_lds(int m, int n, int k, T alpha, BatchArgO<T> A, BatchArgO<T> B, T beta,
         if (m <= 0 || n <= 0 || I0 >= m || J0 >= n) return;
     }
     const int wr = 32 * (wave & 1), wc = 32 * (wave >> 1);   // this wavefront's quarter
+    // SYRK: the diagonal tile's quarter beyond the diagonal has nothing to do
+    const bool idle = syrk && (upper ? I0 + wr > J0 + wc : I0 + wr < J0 + wc);
     const T* Ap = A.get(mat);
     const T* Bp = B.get(mat);
     T* Cp = C.get(mat);
@@ -264,18 +266,20 @@ k_gemm_lds(int m, int n, int k, T alpha, BatchArgO<T> A, BatchArgO<T> B, T beta,
             const int cur = q & 1;
             const bool more = q + 1 < nq;
             if (more) gl_load<T, TA, TB>(Ap, lda, Bp, ldb, m, n, k, I0, J0, (q + 1) * GL_KC, tid, ra, rb);
+            if (!idle) {
 #pragma unroll
-            for (int s2 = 0; s2 < GL_KC / 4; ++s2) {
-                const int kk = 4 * s2 + lg;
-                T fa[2], fb[2];
+                for (int s2 = 0; s2 < GL_KC / 4; ++s2) {
+                    const int kk = 4 * s2 + lg;
+                    T fa[2], fb[2];
 #pragma unroll
-                for (int x = 0; x < 2; ++x) fa[x] = sA[cur][kk][wr + 16 * x + li];
+                    for (int x = 0; x < 2; ++x) fa[x] = sA[cur][kk][wr + 16 * x + li];
 #pragma unroll
-                for (int y = 0; y < 2; ++y) fb[y] = sB[cur][kk][wc + 16 * y + li];
+                    for (int y = 0; y < 2; ++y) fb[y] = sB[cur][kk][wc + 16 * y + li];
 #pragma unroll
-                for (int x = 0; x < 2; ++x)
+                    for (int x = 0; x < 2; ++x)
 #pragma unroll
-                    for (int y = 0; y < 2; ++y) acc[x][y] = mfma16x16x4(fb[y], fa[x], acc[x][y]);
+                        for (int y = 0; y < 2; ++y) acc[x][y] = mfma16x16x4(fb[y], fa[x], acc[x][y]);
+                }
             }
             // the next chunk's values are used only after this chunk's products
             __builtin_amdgcn_sched_barrier(0);
@@ -360,9 +364,17 @@ int gm_dispatch(int ta, int tb, int m, int n, int k, T alpha, kb_mat_t A, kb_mat
 {
     if (m <= 16 || n <= 16) return gm_trans<T, 16>(ta, tb, m, n, k, alpha, A, B, beta, C,
         batch, syrk, upper, vm, vn, vk, skip, s);
-    // SYRK keeps the wavefront tiles: they skip the quarters above the diagonal,
-    // which a 64 x 64 workgroup tile computes and discards (measured slower)
-    if (syrk || m < GM_LDS_MIN || n < GM_LDS_MIN)
+    // SYRK on the workgroup tiles where their padding to 64 costs nothing over the
+    // wavefront tiles' padding to 32 (an even number of 32s): with an odd one they
+    // do 1.3 to 1.7 times the products.  Batch of 2,000 to 20,000, wavefront ->
+    // workgroup tiles, FP32: n = 64 274 -> 237 us, n = 100, k = 30 242 -> 194, n =
+    // 256, k = 16 273 -> 178, k = 256 731 -> 621, but n = 96 265 -> 310; FP64, bound
+    // by the matrix cores either way: n = 256 1,057 -> 1,014 but n = 64 364 -> 394,
+    // n = 128 714 -> 705.  (Non-uniform batches keep the wavefront tiles: their
+    // orders differ from the bound.)
+    const bool even = (((m + 31) / 32) & 1) == 0;
+    const bool sy_lds = !vm && even && m >= GM_LDS_MIN && (sizeof(T) == 4 || m > 192);
+    if ((syrk && !sy_lds) || m < GM_LDS_MIN || n < GM_LDS_MIN)
         return gm_trans<T, 32>(ta, tb, m, n, k, alpha, A, B, beta, C, batch, syrk, upper, vm, vn, vk, skip, s);
     return gm_trans<T, GL_TM>(ta, tb, m, n, k, alpha, A, B, beta, C, batch, syrk, upper, vm, vn, vk, skip, s);
 }

@@ -223,3 +223,12 @@ def test_gemm_workgroup_tiles_alpha_zero_reads_no_operands(h):
                                         -1.5, kt.P(dC), m, m * n, batch)
     assert st == pykblas.KBLAS_Success
     assert np.array_equal(kt.to_host(dC), -1.5 * C)
+
+
+@pytest.mark.parametrize("p", ["D", "S"])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("upper", [False, True])
+@pytest.mark.parametrize("mk", [(64, 1), (64, 65), (97, 33), (127, 16), (128, 40), (161, 15), (193, 17), (255, 31), (256, 64)])
+def test_syrk_workgroup_tiles(h, p, trans, upper, mk):
+    """SYRK at the orders that may take 64 x 64 workgroup tiles, and beside them"""
+    test_syrk(h, p, trans, upper, mk)
