@@ -190,6 +190,22 @@ KB_DEV void rg_solve(const T (&a)[NB / 16][NB], const T (&dinv2)[NB / 16], const
     }
 }
 
+// right-hand sides c0 .. c0 + RC - 1 (zero beyond nrhs and n)
+template <typename T, int NB, int RC, bool EX>
+KB_DEV void rg_rhs(T (&x)[RC][NB / 16], T* Bp, int ldb, int side_left, int n, int nrhs, int c0, int l)
+{
+#pragma unroll
+    for (int s = 0; s < NB / 16; ++s) {
+        const int i = 16 * s + l;
+#pragma unroll
+        for (int c = 0; c < RC; ++c) {
+            const bool in = (EX || i < n) && c0 + c < nrhs;
+            const T v = gld(rhs_elem(Bp, ldb, side_left, in ? i : 0, in ? c0 + c : 0));
+            x[c][s] = in ? v : T(0);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // one matrix per 16-lane row; WPB wavefronts (4 WPB matrices) per workgroup
 // ---------------------------------------------------------------------------
@@ -217,6 +233,11 @@ k_rg_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* inf
 #pragma unroll
     for (int s = 0; s < R; ++s) dinv2[s] = T(1);
     rg_load<T, NB, EX>(a, Ap, lda, n, l);
+    // POTRS: the first right-hand sides go out with the factor, so the call waits
+    // for memory once (POSV's registers are full during the factorization)
+    constexpr bool EARLY = MODE == KB_MODE_POTRS;
+    T x0[EARLY ? RC : 1][R];
+    if constexpr (EARLY) rg_rhs<T, NB, RC, EX>(x0, B.get(m), B.ldim(m), side_left, n, nrhs, 0, l);
 
     int inf = 0;
     if constexpr (MODE != KB_MODE_POTRS) {
@@ -242,15 +263,13 @@ k_rg_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* inf
         const bool ok = live && inf == 0;
         for (int c0 = 0; c0 < nrhs; c0 += RC) {
             T x[RC][R];
+            if (EARLY && c0 == 0) {
 #pragma unroll
-            for (int s = 0; s < R; ++s) {
-                const int i = 16 * s + l;
+                for (int c = 0; c < RC; ++c)
 #pragma unroll
-                for (int c = 0; c < RC; ++c) {
-                    const bool in = (EX || i < n) && c0 + c < nrhs;
-                    const T v = gld(rhs_elem(Bp, ldb, side_left, in ? i : 0, in ? c0 + c : 0));
-                    x[c][s] = in ? v : T(0);
-                }
+                    for (int s = 0; s < R; ++s) x[c][s] = x0[EARLY ? c : 0][s];
+            } else {
+                rg_rhs<T, NB, RC, EX>(x, Bp, ldb, side_left, n, nrhs, c0, l);
             }
             rg_solve<T, NB, RC>(a, dinv2, Lt, x, l);
 #pragma unroll
