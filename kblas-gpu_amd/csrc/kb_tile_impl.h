@@ -32,13 +32,14 @@
 
 constexpr KB_DEV int tix(int I, int J) { return I * (I + 1) / 2 + J; }
 
-// Per-wave LDS: a 64 x 4 panel transpose buffer and a 16 x 17 tile staging buffer.
-template <typename T>
+// Per-wave LDS: a 64 x 4 panel transpose buffer and a 16 x 17 tile staging buffer;
+// NG groups of four right-hand sides.
+template <typename T, int NG>
 struct TileLds {
     T pan[4][16][4];
     T tile[16][17];
     T inv[16];
-    T y[4][64];      // right-hand-side blocks during the solve
+    T y[NG][4][64];  // right-hand-side blocks during the solve
     T invd[4][64];   // 1/L(16K+i,16K+i) per lane
 };
 
@@ -175,8 +176,8 @@ KB_DEV int tile_potrf(typename TileV<T>::v4 (&t)[NT * (NT + 1) / 2], T (&invd)[N
 // the unit factor Lu = L D^-1 (column c scaled by 1/L(c,c); invk = this lane's
 // 1/L(i,i)): row i gives Lu(i, j), column i gives Lu(j, i), so the sweeps need
 // no per-step division.
-template <typename T, bool ROW, bool STRICT>
-KB_DEV void tile_stage(const T* L, int lda, int n, int I, int J, T (&v)[16], TileLds<T>& S, int lane,
+template <typename T, bool ROW, bool STRICT, int NG>
+KB_DEV void tile_stage(const T* L, int lda, int n, int I, int J, T (&v)[16], TileLds<T, NG>& S, int lane,
                        T invk = T(1))
 {
     const int i = lane & 15, g = lane >> 4;
@@ -201,11 +202,11 @@ KB_DEV void tile_stage(const T* L, int lda, int n, int I, int J, T (&v)[16], Til
 }
 
 // Factor tiles read from L in global memory (staged through LDS).
-template <typename T>
+template <typename T, int NG>
 struct GlobalTiles {
     const T* L;
     int lda, n;
-    TileLds<T>* S;
+    TileLds<T, NG>* S;
     template <bool ROW, bool STRICT>
     KB_DEV void get(int I, int J, T (&v)[16], int lane, T invk) const
     {
@@ -215,10 +216,10 @@ struct GlobalTiles {
 
 // Factor tiles taken from the wavefront's registers (the factorization's
 // output, or a tile_load of L), staged through LDS one tile at a time.
-template <typename T>
+template <typename T, int NG>
 struct RegTiles {
     const typename TileV<T>::v4* t;
-    TileLds<T>* S;
+    TileLds<T, NG>* S;
     template <bool ROW, bool STRICT>
     KB_DEV void get(int I, int J, T (&v)[16], int lane, T invk) const
     {
@@ -253,33 +254,43 @@ struct RegTiles {
     }
 };
 
-// (L L^T) X = B for the group's four right-hand sides.  Right-hand side c of
-// the group sits in DPP row c: y[K][16c + i] = row 16K + i.  The tile loops
+// (L L^T) X = B for NG groups of four right-hand sides.  Right-hand side c of
+// group q sits in DPP row c: y[q][K][16c + i] = row 16K + i.  The tile loops
 // are runtime loops over LDS-resident blocks so that register use stays that
 // of a single 16 x 16 step.  src.get<ROW,STRICT>(I, J, v, lane, 1/L(i,i))
 // returns row / column i of factor tile (I,J) (STRICT: unit-scaled strictly
 // lower part of a diagonal tile).
-template <typename T, typename Src>
-KB_DEV void tile_solve(const Src& src, T (&y)[4][64], const T (&invd)[4][64], int lane)
+template <typename T, int NG, typename Src>
+KB_DEV void tile_solve(const Src& src, T (&y)[NG][4][64], const T (&invd)[4][64], int lane)
 {
-    T v[16];
+    T v[16], yk[NG], yi[NG];
     // forward: L y = b, L = Lu D with Lu unit lower: z = Lu^-1 b, y = D^-1 z
 #pragma nounroll
     for (int K = 0; K < 4; ++K) {
         const T ik = invd[K][lane];
-        T yk = y[K][lane];
+#pragma unroll
+        for (int q = 0; q < NG; ++q) yk[q] = y[q][K][lane];
         src.template get<true, true>(K, K, v, lane, ik);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) fnmac_rowk<T>(yk, yk, v[j], j);
-        yk *= ik;
-        y[K][lane] = yk;
+        for (int j = 0; j < 16; ++j)
+#pragma unroll
+            for (int q = 0; q < NG; ++q) fnmac_rowk<T>(yk[q], yk[q], v[j], j);
+#pragma unroll
+        for (int q = 0; q < NG; ++q) {
+            yk[q] *= ik;
+            y[q][K][lane] = yk[q];
+        }
 #pragma nounroll
         for (int I = K + 1; I < 4; ++I) {
-            T yi = y[I][lane];
+#pragma unroll
+            for (int q = 0; q < NG; ++q) yi[q] = y[q][I][lane];
             src.template get<true, false>(I, K, v, lane, T(1));
 #pragma unroll
-            for (int j = 0; j < 16; ++j) fnmac_rowk<T>(yi, yk, v[j], j);
-            y[I][lane] = yi;
+            for (int j = 0; j < 16; ++j)
+#pragma unroll
+                for (int q = 0; q < NG; ++q) fnmac_rowk<T>(yi[q], yk[q], v[j], j);
+#pragma unroll
+            for (int q = 0; q < NG; ++q) y[q][I][lane] = yi[q];
         }
     }
     // backward: L^T x = y; on the diagonal tile L^T = D Lu^T, so scale by
@@ -287,30 +298,58 @@ KB_DEV void tile_solve(const Src& src, T (&y)[4][64], const T (&invd)[4][64], in
 #pragma nounroll
     for (int K = 3; K >= 0; --K) {
         const T ik = invd[K][lane];
-        T yk = y[K][lane];
+#pragma unroll
+        for (int q = 0; q < NG; ++q) yk[q] = y[q][K][lane];
 #pragma nounroll
         for (int I = K + 1; I < 4; ++I) {
-            const T xi = y[I][lane];
+#pragma unroll
+            for (int q = 0; q < NG; ++q) yi[q] = y[q][I][lane];
             src.template get<false, false>(I, K, v, lane, T(1));
 #pragma unroll
-            for (int j = 0; j < 16; ++j) fnmac_rowk<T>(yk, xi, v[j], j);
+            for (int j = 0; j < 16; ++j)
+#pragma unroll
+                for (int q = 0; q < NG; ++q) fnmac_rowk<T>(yk[q], yi[q], v[j], j);
         }
         src.template get<false, true>(K, K, v, lane, ik);
-        yk *= ik;
 #pragma unroll
-        for (int j = 15; j >= 0; --j) fnmac_rowk<T>(yk, yk, v[j], j);
-        y[K][lane] = yk;
+        for (int q = 0; q < NG; ++q) yk[q] *= ik;
+#pragma unroll
+        for (int j = 15; j >= 0; --j)
+#pragma unroll
+            for (int q = 0; q < NG; ++q) fnmac_rowk<T>(yk[q], yk[q], v[j], j);
+#pragma unroll
+        for (int q = 0; q < NG; ++q) y[q][K][lane] = yk[q];
     }
 }
 
-template <typename T, int MODE>
+// right-hand sides c0 + 4 q + c (zero beyond nrhs and n), in tile_solve's layout
+template <typename T, int NG>
+KB_DEV void tile_rhs(T (&v)[NG][4], T* Bp, int ldb, int side_left, int n, int nrhs, int c0, int lane)
+{
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+        const int c = c0 + 4 * q + (lane >> 4);
+#pragma unroll
+        for (int K = 0; K < 4; ++K) {
+            const int row = 16 * K + (lane & 15);
+            const bool in = c < nrhs && row < n;
+            const T x = gld(rhs_elem(Bp, ldb, side_left, in ? row : 0, in ? c : 0));
+            v[q][K] = in ? x : T(0);
+        }
+    }
+}
+
+template <typename T, int MODE, int NG>
 KB_DEV void tile_chol_one(int n, int nrhs, int side_left, T* Ap, int lda, T* Bp, int ldb, int* info_out,
-                          TileLds<T>& S, int lane)
+                          TileLds<T, NG>& S, int lane)
 {
     T invd[4] = {T(1), T(1), T(1), T(1)};
     int inf = 0;
     const int i = lane & 15;
     typename TileV<T>::v4 t[10];
+    // the first right-hand sides go out with the matrix: one wait for memory
+    T v[NG][4];
+    if constexpr (MODE != KB_MODE_POTRF) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, 0, lane);
     if constexpr (MODE != KB_MODE_POTRS) {
         tile_load<T>(t, Ap, lda, n, lane);
         inf = tile_potrf<T>(t, invd, n, S.pan, lane);
@@ -329,41 +368,41 @@ KB_DEV void tile_chol_one(int n, int nrhs, int side_left, T* Ap, int lda, T* Bp,
         if (inf) return;
 #pragma unroll
         for (int K = 0; K < 4; ++K) S.invd[K][lane] = invd[K];
-        const int c = lane >> 4;
-        for (int c0 = 0; c0 < nrhs; c0 += 4) {
-            const bool act = c0 + c < nrhs;
+        for (int c0 = 0; c0 < nrhs; c0 += 4 * NG) {
+            if (c0 > 0) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, c0, lane);
 #pragma unroll
-            for (int K = 0; K < 4; ++K) {
-                const int row = 16 * K + i;
-                const bool in = act && row < n;
-                const T ld = gld(rhs_elem(Bp, ldb, side_left, in ? row : 0, in ? c0 + c : 0));
-                S.y[K][lane] = in ? ld : T(0);
-            }
+            for (int q = 0; q < NG; ++q)
+#pragma unroll
+                for (int K = 0; K < 4; ++K) S.y[q][K][lane] = v[q][K];
             wave_lds_sync();
-            RegTiles<T> src{t, &S};
-            tile_solve<T>(src, S.y, S.invd, lane);
+            RegTiles<T, NG> src{t, &S};
+            tile_solve<T, NG>(src, S.y, S.invd, lane);
             wave_lds_sync();
 #pragma unroll
-            for (int K = 0; K < 4; ++K) {
-                const int row = 16 * K + i;
-                if (act && row < n) gst(rhs_elem(Bp, ldb, side_left, row, c0 + c), S.y[K][lane]);
+            for (int q = 0; q < NG; ++q) {
+                const int c = c0 + 4 * q + (lane >> 4);
+#pragma unroll
+                for (int K = 0; K < 4; ++K) {
+                    const int row = 16 * K + i;
+                    if (c < nrhs && row < n) gst(rhs_elem(Bp, ldb, side_left, row, c), S.y[q][K][lane]);
+                }
             }
         }
     }
 }
 
 // 4 wavefronts (4 matrices) per 256-thread workgroup
-template <typename T, int MODE>
+template <typename T, int MODE, int NG>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
 k_tile_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* info, int batch)
 {
-    __shared__ TileLds<T> S[4];
+    __shared__ TileLds<T, NG> S[4];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const long mat = (long)blockIdx.x * 4 + wave;
     if (mat >= batch) return;
     T* Bp = (MODE == KB_MODE_POTRF) ? nullptr : B.get(mat);
     const int ldb = (MODE == KB_MODE_POTRF) ? 1 : B.ldim(mat);
-    tile_chol_one<T, MODE>(n, nrhs, side_left, A.get(mat), A.ldim(mat), Bp, ldb, info ? info + mat : nullptr,
+    tile_chol_one<T, MODE, NG>(n, nrhs, side_left, A.get(mat), A.ldim(mat), Bp, ldb, info ? info + mat : nullptr,
                            S[wave], lane);
 }
 
@@ -373,12 +412,16 @@ static int launch_tile(int mode, int n, int nrhs, int side_left, kb_mat_t A, kb_
 {
     dim3 grid((unsigned)((batch + 3) / 4));
     BatchArg<T> a = to_arg<T>(A), b = to_arg<T>(B);
+    // two groups of four right-hand sides share each staged factor tile
     if (mode == KB_MODE_POTRF)
-        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POTRF>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
+        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POTRF, 1>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
+    else if (mode == KB_MODE_POSV && nrhs <= 4)
+        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POSV, 1>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
     else if (mode == KB_MODE_POSV)
-        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POSV>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
+        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POSV, 2>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
+    else if (nrhs <= 4)
+        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POTRS, 1>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
     else
-        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POTRS>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
+        hipLaunchKernelGGL((k_tile_chol<T, KB_MODE_POTRS, 2>), grid, dim3(256), 0, s, n, nrhs, side_left, a, b, info, batch);
     return (int)hipGetLastError();
 }
-

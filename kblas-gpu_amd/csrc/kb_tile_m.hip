@@ -22,7 +22,7 @@ struct MixLds {
             float d2[4][64];          // 1/L32(16K+i, 16K+i)^2 per lane
             double tile[16][17];      // FP64 tile transposes, then the solution blocks of the residual
         } m;
-        TileLds<double> d;            // FP64 fallback
+        TileLds<double, 1> d;          // FP64 fallback
     };
 };
 
@@ -417,16 +417,16 @@ k_tile_sposv(int n, int nrhs, int side_left, BatchArg<double> A, BatchArg<double
                     const int row = 16 * K + i;
                     const bool in = act && row < n;
                     const double ld = gld(rhs_elem(Bp, ldb, side_left, in ? row : 0, in ? c0 + c : 0));
-                    S.d.y[K][lane] = in ? ld : 0.0;
+                    S.d.y[0][K][lane] = in ? ld : 0.0;
                 }
                 wave_lds_sync();
-                GlobalTiles<double> src{Ap, lda, n, &S.d};
-                tile_solve<double>(src, S.d.y, S.d.invd, lane);
+                GlobalTiles<double, 1> src{Ap, lda, n, &S.d};
+                tile_solve<double, 1>(src, S.d.y, S.d.invd, lane);
                 wave_lds_sync();
 #pragma unroll
                 for (int K = 0; K < 4; ++K) {
                     const int row = 16 * K + i;
-                    if (act && row < n) gst(rhs_elem(Xp, ldx, side_left, row, c0 + c), S.d.y[K][lane]);
+                    if (act && row < n) gst(rhs_elem(Xp, ldx, side_left, row, c0 + c), S.d.y[0][K][lane]);
                 }
             }
         }

@@ -94,3 +94,12 @@ def test_potrs_wide_uses_given_factor(h, side, n):
     for i in range(batch):
         Xo = po.potrs(side, po.col(Lh, i), po.col(B, i))
         assert np.max(np.abs(po.col(X, i) - Xo)) <= 64 * n * kt.EPS64 * max(np.max(np.abs(Xo)), 1)
+
+
+@pytest.mark.parametrize("p", ["D", "S"])
+@pytest.mark.parametrize("side", ["L", "R"])
+@pytest.mark.parametrize("n,nrhs", [(33, 5), (40, 8), (47, 9), (50, 4), (63, 16), (64, 13), (64, 31)])
+def test_posv_pairs_of_groups(h, p, side, n, nrhs):
+    """5 to 31 right-hand sides at orders 33..64: two groups of four share a
+    pass, the last one partly empty or with its second group empty"""
+    test_posv_wide(h, p, side, n, nrhs)
