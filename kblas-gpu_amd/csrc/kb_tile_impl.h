@@ -349,7 +349,10 @@ KB_DEV void tile_chol_one(int n, int nrhs, int side_left, T* Ap, int lda, T* Bp,
     typename TileV<T>::v4 t[10];
     // the first right-hand sides go out with the matrix: one wait for memory
     T v[NG][4];
-    if constexpr (MODE != KB_MODE_POTRF) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, 0, lane);
+    if constexpr (MODE != KB_MODE_POTRF) {
+        // (POSV without right-hand sides only factors: B may not exist)
+        if (nrhs > 0) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, 0, lane);
+    }
     if constexpr (MODE != KB_MODE_POTRS) {
         tile_load<T>(t, Ap, lda, n, lane);
         inf = tile_potrf<T>(t, invd, n, S.pan, lane);

@@ -103,3 +103,23 @@ def test_posv_pairs_of_groups(h, p, side, n, nrhs):
     """5 to 31 right-hand sides at orders 33..64: two groups of four share a
     pass, the last one partly empty or with its second group empty"""
     test_posv_wide(h, p, side, n, nrhs)
+
+
+@pytest.mark.parametrize("n", [12, 30, 50, 64, 100])
+def test_posv_without_right_hand_sides_only_factors(h, n):
+    """0 right-hand sides: A := L, and B, which has no elements, is not read
+    (its pointers are null)"""
+    torch = kt.torch_dev()
+    batch = 6
+    A = po.gen_spd_shift_batch(80 + n, n, batch)
+    dA = kt.to_dev(nan_upper(A))
+    pA = kt.ptr_array(dA, batch, n * n)
+    pB = torch.zeros(batch, dtype=torch.int64, device="cuda")
+    info = kt.to_dev(np.full(batch, -7, np.int32))
+    st = h.lib.kblasDposv_batch(h.h, b"R", b"L", 0, n, kt.P(pA), n, kt.P(pB), 1, batch, kt.P(info))
+    assert st == pykblas.KBLAS_Success
+    assert np.all(kt.to_host(info) == 0)
+    for i in range(batch):
+        Lo, _ = po.potrf(po.col(A, i))
+        got = np.tril(po.col(kt.to_host(dA), i))
+        assert np.max(np.abs(got - np.tril(Lo))) <= 64 * n * kt.EPS64 * np.max(np.abs(Lo))
