@@ -16,12 +16,12 @@
 //   - right-hand sides (POSV) are further row tiles of the panel: the forward
 //     sweep L Y = B is the panel solve Y^T = B^T L^-T.
 // What bounds it: the serial chain of a panel (the loads' latency, the 32
-// pivots, two barriers), hidden by four workgroups per CU.  Against the
-// right-looking form it replaces (trailing matrix read and written once per 64
-// columns, rows solved by substitution one per thread): DPOTRF n = 200 x 2,000
-// 725 -> 350 us, n = 256 x 4,096 1.82 -> 0.86 ms, n = 128 x 8,000 0.82 -> 0.45
-// ms; the workgroup phase of the non-uniform DPOSV of orders 8..256 x 20,000
-// 4.50 -> 2.65 ms.
+// pivots, two barriers), hidden by the four or eight workgroups of a CU.  Against
+// the right-looking form it replaces (trailing matrix read and written once per
+// 64 columns, rows solved by substitution one per thread): DPOTRF n = 200 x
+// 2,000 725 -> 300 us, n = 256 x 4,096 1.82 -> 0.85 ms, n = 128 x 8,000 0.82 ->
+// 0.32 ms; the workgroup phase of the non-uniform DPOSV of orders 8..256 x
+// 20,000 4.69 -> 2.82 ms.
 // The solve (POSV/POTRS) runs blocked forward and backward sweeps over up to
 // 64 right-hand sides per pass (so L is streamed once per sweep for up to 64
 // right-hand sides): the diagonal blocks by DPP-row substitutions, the

@@ -23,7 +23,7 @@
 // matrix-core layout: lane (c, g) holds rows 4g..4g+3 of right-hand side c, so
 // a tile is one 16-byte access per lane, and a product's result is the next
 // product's operand.  On 2,000 systems of order 128..512 with 64 right-hand
-// sides: 5.7 ms, where sweeps shared by the waves (two barriers per 32 rows, the
+// sides: 5.6 ms, where sweeps shared by the waves (two barriers per 32 rows, the
 // right-hand sides updated in memory at each) and a residual staging X in LDS
 // took 13.7 ms.
 #pragma once
