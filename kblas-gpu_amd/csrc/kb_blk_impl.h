@@ -10,7 +10,8 @@
 //     registers (4-column panels on DPP rows, rank-4 updates on the matrix
 //     cores) and leaves the inverses of the two 16x16 diagonal tiles in LDS;
 //   - meanwhile waves 1..3 read the 16-row tiles below and subtract the same
-//     products, then solve them against the inverses, all in registers: every
+//     products, then solve them against the inverses (with a correction step
+//     where a diagonal tile is ill-conditioned), all in registers: every
 //     element of A is read once and every element of L written once, and the
 //     only other traffic is re-reading finished columns of L;
 //   - right-hand sides (POSV) are further row tiles of the panel: the forward
@@ -61,6 +62,7 @@ struct BlkSmem {
     };
     T sInv[KB_BLK_NBK];
     int flag;
+    int grow;   // bit 0: the factored panel has an ill-conditioned diagonal tile (KB_LL_GROW)
 };
 
 // B(i, c) of a right-hand-side block: side_left -> column c, else row c.
@@ -379,6 +381,16 @@ template <typename T> constexpr int ll_step(int e) { return sizeof(T) == 8 ? 4 :
 constexpr int KB_LL_U = 1;
 constexpr int KB_LL_KC = 64;   // columns whose products are summed before they are taken from C
 
+// A diagonal tile L counts as ill-conditioned when four columns of W = L^-1 give a
+// row of |W| |L| (unchanged by a scaling of A's rows and columns) more than this,
+// or a NaN; its row sums stay below 16 otherwise.  B B^T + n I of order 200 has
+// sums of 1.6, Q diag(s) Q^T of condition 1e4 up to 10, a Gaussian kernel matrix
+// at the limit of FP64 1e6: without the correction POTRF's error there is 1,000
+// times substitution's, or a pivot comes out negative.  Forming the measure is in
+// wave 0's serial part: DPOTRF n = 200, one matrix, 87.7 -> 88.7 us, SPOTRF 66.9 ->
+// 68.3 us, batches that fill the chip as before.
+constexpr int KB_LL_GROW = 4;
+
 // c[j] := C_j - L_j L_P^T in transposed form for NT tiles: register r of column
 // block q holds, in lane (i, g), row i and panel column 16 q + blk_drow(r, g).
 // Lp: the panel's rows of L (row k0, column 0), kb of them valid; rows and
@@ -459,21 +471,34 @@ KB_DEV void ll_update(const T* Lp, int lda, int kb, int k0, const LlTile<T>* t, 
     }
 }
 
-// W c for the inverse W of a 16 x 16 triangle
+// x + W c for the inverse W of a 16 x 16 triangle
 template <typename T>
-KB_DEV typename TileV<T>::v4 ll_apply(const T* W, int li, int lg, const typename TileV<T>::v4& c)
+KB_DEV typename TileV<T>::v4 ll_apply(const T* W, int li, int lg, const typename TileV<T>::v4& c,
+                                      typename TileV<T>::v4 x = {T(0), T(0), T(0), T(0)})
 {
-    typename TileV<T>::v4 x = {T(0), T(0), T(0), T(0)};
 #pragma unroll
     for (int s = 0; s < 4; ++s) x = mfma16x16x4(W[li * KB_LL_LD + blk_drow<T>(s, lg)], c[s], x);
     return x;
+}
+
+// c - L x for the 16 x 16 triangle L (zero above its diagonal) at L, pitch LD
+template <typename T, int LD>
+KB_DEV typename TileV<T>::v4 ll_resid(const T* L, int li, int lg, const typename TileV<T>::v4& x,
+                                      typename TileV<T>::v4 c)
+{
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c = mfma16x16x4(-L[li * LD + blk_drow<T>(s, lg)], x[s], c);
+    return c;
 }
 
 // One updated tile solved against the factored diagonal block and stored:
 // X1^T = L11^-1 C1^T, X2^T = L22^-1 (C2^T - L21 X1^T).  A 16 x 16 accumulator is
 // itself the second operand of the next product (register s of lane group g
 // holds row kmap(s, g)), so nothing leaves the registers.
-template <typename T, int CB>
+// The product W c with an inverse W errs by eps |L| |W| |L| |x|, a substitution by
+// eps |L| |x|: where |W| |L| is large (COR, see KB_LL_GROW) one correction
+// x += W (c - L x) brings the error back to the substitution's.
+template <typename T, int CB, bool COR>
 KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const BlkSmem<T, CB>& S,
                      typename TileV<T>::v4 (&c)[2])
 {
@@ -485,15 +510,29 @@ KB_DEV void ll_solve(const LlTile<T>& t, int kb, int k0, int li, int lg, const B
             if (16 * (e >> 2) + blk_drow<T>(e & 3, lg) >= kb) c[e >> 2][e & 3] = T(0);
     }
     x[0] = ll_apply<T>(S.fW[0], li, lg, c[0]);
+    if (COR) x[0] = ll_apply<T>(S.fW[0], li, lg, ll_resid<T, LD>(S.fD, li, lg, x[0], c[0]), x[0]);
 #pragma unroll
     for (int s = 0; s < 4; ++s) c[1] = mfma16x16x4(-S.fD[(16 + li) * LD + blk_drow<T>(s, lg)], x[0][s], c[1]);
     x[1] = ll_apply<T>(S.fW[1], li, lg, c[1]);
+    if (COR)
+        x[1] = ll_apply<T>(S.fW[1], li, lg, ll_resid<T, LD>(S.fD + 16 * LD + 16, li, lg, x[1], c[1]), x[1]);
     T* p = t.p + (long)li * t.rs + (k0 + blk_drow<T>(0, lg)) * t.cs;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         if (li < t.rows && 16 * (e >> 2) + blk_drow<T>(e & 3, lg) < kb) gst(p, x[e >> 2][e & 3]);
         p += ll_step<T>(e) * t.cs;
         asm volatile("" : "+v"(p));
+    }
+}
+
+template <typename T, int NT, int CB, bool COR>
+KB_DEV void ll_solve_n(const LlTile<T>* t, int kb, int k0, int li, int lg, const BlkSmem<T, CB>& S,
+                       typename TileV<T>::v4 (&c)[NT][2])
+{
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        ll_solve<T, CB, COR>(t[j], kb, k0, li, lg, S, c[j]);
+        __builtin_amdgcn_sched_barrier(0);   // one tile's products at a time (registers)
     }
 }
 
@@ -506,20 +545,15 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
 {
     typename TileV<T>::v4 c[NT > 0 ? NT : 1][2];
     if constexpr (NT > 0) ll_update<T, NT>(Lp, lda, kb, k0, t, li, lg, c);
-    if (first) {
-        __syncthreads();
-        const int f = S.flag;
-        if (f) return f;
-    }
+    if (first) __syncthreads();
+    const int f = uniform(S.flag), grow = uniform(S.grow);   // (one wait for both)
+    if (first && f) return f;
     if constexpr (NT > 0) {
         // formed here, not kept live (or as induction variables) across panels
         asm volatile("" : "+v"(li), "+v"(lg));
         asm volatile("" : "+s"(k0));
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            ll_solve<T, CB>(t[j], kb, k0, li, lg, S, c[j]);
-            __builtin_amdgcn_sched_barrier(0);   // one tile's products at a time (registers)
-        }
+        if (grow & 1) ll_solve_n<T, NT, CB, true>(t, kb, k0, li, lg, S, c);
+        else ll_solve_n<T, NT, CB, false>(t, kb, k0, li, lg, S, c);
     }
     return 0;
 }
@@ -626,6 +660,15 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
                 if (row < kb && col <= row) gst(D + row + (long)col * lda, c[tix(I, J)][r]);
                 S.fD[row * LD + col] = (col <= row) ? c[tix(I, J)][r] : T(0);
             }
+    // the row sums of the diagonal tiles' |L|
+    T* rs = &S.tpan[0][0][0];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        T v = T(0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v += (4 * g + r <= i) ? kb_abs<T>(c[tix(b, b)][r]) : T(0);
+        rs[16 * b + i] = sum_rows4<T>(v);
+    }
     if (g == 0) {
         S.sInv[i] = invd[0];
         S.sInv[16 + i] = invd[1];
@@ -634,7 +677,11 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
     wave_lds_sync();
     // the inverses of both diagonal tiles: DPP row g takes columns 4g..4g+3 of
     // each, lane i of the row holds their row i
-    T y[2][4];
+    T y[2][4], lsum[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) lsum[b][s] = rs[16 * b + 4 * g + s];
 #pragma unroll
     for (int s = 0; s < 4; ++s) y[0][s] = y[1][s] = (i == 4 * g + s) ? T(1) : T(0);
 #pragma unroll
@@ -647,14 +694,20 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
             for (int s = 0; s < 4; ++s) fnmac_rowk<T>(y[b][s], y[b][s] * ij, l, j);
         }
     }
+    int grow = 0;
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 2; ++b) {
+        T m = T(0);   // this lane's four columns' part of a row of |W| |L| (its sum)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const T v = y[b][s] * S.sInv[16 * b + i];
             S.fW[b][i * KB_LL_LD + 4 * g + s] = v;
             if (W && 16 * b < kb) gst(W + 16L * (k0 + 16 * b) + 16 * i + 4 * g + s, v);
+            m += kb_abs<T>(v) * lsum[b][s];
         }
+        if (__any(!(m <= T(KB_LL_GROW)))) grow |= 1;
+    }
+    if (lane == 0) S.grow = grow;
 }
 
 // In-place lower Cholesky of an n x n matrix by the whole workgroup.
@@ -731,9 +784,15 @@ KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T, CB>& S, T* B = nullptr, in
 }
 
 // CB = 2: passes of 32 right-hand sides, few enough registers for four
-// waves per SIMD; CB = 4: passes of 64 (L streamed half as often), three.
+// waves per SIMD (FP32 POTRF: five, SPOTRF n = 256 x 1,100 177 us, with four 231);
+// CB = 4: passes of 64 (L streamed half as often), three.
+template <typename T, int MODE, int CB> constexpr int blk_wpe()
+{
+    return CB != 2 ? 2 : sizeof(T) == 4 && MODE == KB_MODE_POTRF ? 5 : 4;
+}
+
 template <typename T, int MODE, int CB, int W>
-__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(CB == 2 ? 4 : 2)))
+__global__ void __launch_bounds__(W) __attribute__((amdgpu_waves_per_eu(blk_wpe<T, MODE, CB>())))
 k_blk_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* info, int batch)
 {
     __shared__ BlkSmem<T, CB> S;

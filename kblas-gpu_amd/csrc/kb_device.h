@@ -375,6 +375,33 @@ template <> KB_DEV float kb_rcp<float>(float x)
     return __builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r);
 }
 
+template <typename T> KB_DEV T kb_abs(T x);
+template <> KB_DEV double kb_abs<double>(double x) { return __builtin_fabs(x); }
+template <> KB_DEV float kb_abs<float>(float x) { return __builtin_fabsf(x); }
+
+// Sum of v over the four lanes of the wave that share lane % 16 (exchanges by
+// vector instructions, no LDS round trip): the two halves first, then the two
+// rows of 16 of each half.
+template <typename T>
+KB_DEV T sum_rows4(T v)
+{
+    struct W { unsigned w[sizeof(T) / 4]; };
+#pragma unroll
+    for (int step = 0; step < 2; ++step) {
+        const W x = __builtin_bit_cast(W, v);
+        W a, b;
+#pragma unroll
+        for (unsigned q = 0; q < sizeof(T) / 4; ++q) {
+            const auto r = step == 0 ? __builtin_amdgcn_permlane32_swap(x.w[q], x.w[q], false, false)
+                                     : __builtin_amdgcn_permlane16_swap(x.w[q], x.w[q], false, false);
+            a.w[q] = r[0];
+            b.w[q] = r[1];
+        }
+        v = __builtin_bit_cast(T, a) + __builtin_bit_cast(T, b);
+    }
+    return v;
+}
+
 template <typename T> KB_DEV T kb_sqrt(T x);
 template <> KB_DEV double kb_sqrt<double>(double x) { return __builtin_sqrt(x); }
 template <> KB_DEV float kb_sqrt<float>(float x) { return __builtin_sqrtf(x); }
