@@ -62,7 +62,7 @@ struct BlkSmem {
     };
     T sInv[KB_BLK_NBK];
     int flag;
-    int grow;   // bit 0: the factored panel has an ill-conditioned diagonal tile (KB_LL_GROW)
+    int grow;   // KB_GROW_* bits
 };
 
 // B(i, c) of a right-hand-side block: side_left -> column c, else row c.
@@ -390,6 +390,13 @@ constexpr int KB_LL_KC = 64;   // columns whose products are summed before they 
 // wave 0's serial part: DPOTRF n = 200, one matrix, 87.7 -> 88.7 us, SPOTRF 66.9 ->
 // 68.3 us, batches that fill the chip as before.
 constexpr int KB_LL_GROW = 4;
+// The same for the mixed routine's FP32 sweeps, whose result a refinement corrects:
+// row sums below 128 cost no more than the rounding of a substitution over 65 or
+// more rows, and random matrices of condition 1e4 (2,000 systems of order
+// 128..512: 5.55 ms, with a limit of 4 5.70) stay without the correction.
+constexpr int KB_LL_GROW_SWEEP = 32;
+constexpr int KB_GROW_NOW = 1;   // the factored panel has a tile above KB_LL_GROW
+constexpr int KB_GROW_ANY = 2;   // a panel so far has one above KB_LL_GROW_SWEEP
 
 // c[j] := C_j - L_j L_P^T in transposed form for NT tiles: register r of column
 // block q holds, in lane (i, g), row i and panel column 16 q + blk_drow(r, g).
@@ -552,7 +559,7 @@ KB_DEV int ll_group(bool first, const T* Lp, int lda, int kb, int k0, const LlTi
         // formed here, not kept live (or as induction variables) across panels
         asm volatile("" : "+v"(li), "+v"(lg));
         asm volatile("" : "+s"(k0));
-        if (grow & 1) ll_solve_n<T, NT, CB, true>(t, kb, k0, li, lg, S, c);
+        if (grow & KB_GROW_NOW) ll_solve_n<T, NT, CB, true>(t, kb, k0, li, lg, S, c);
         else ll_solve_n<T, NT, CB, false>(t, kb, k0, li, lg, S, c);
     }
     return 0;
@@ -694,7 +701,7 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
             for (int s = 0; s < 4; ++s) fnmac_rowk<T>(y[b][s], y[b][s] * ij, l, j);
         }
     }
-    int grow = 0;
+    int grow = k0 > 0 ? S.grow & KB_GROW_ANY : 0;
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         T m = T(0);   // this lane's four columns' part of a row of |W| |L| (its sum)
@@ -705,7 +712,10 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
             if (W && 16 * b < kb) gst(W + 16L * (k0 + 16 * b) + 16 * i + 4 * g + s, v);
             m += kb_abs<T>(v) * lsum[b][s];
         }
-        if (__any(!(m <= T(KB_LL_GROW)))) grow |= 1;
+        if (__any(!(m <= T(KB_LL_GROW)))) {
+            grow |= KB_GROW_NOW;
+            if (__any(!(m <= T(KB_LL_GROW_SWEEP)))) grow |= KB_GROW_ANY;
+        }
     }
     if (lane == 0) S.grow = grow;
 }
@@ -716,7 +726,8 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
 // being further row tiles of every panel; a factorization that fails at panel k
 // leaves B forward-solved in the rows of the panels before k and as it was in
 // the others.  Wt, if given, receives the inverses of the factor's 16 x 16
-// diagonal tiles (row-major, identity beyond n).
+// diagonal tiles (row-major, identity beyond n); S.grow then says whether
+// products with them need the correction (KB_GROW_ANY).
 template <typename T, int CB = 4, int W = KB_BLK_WG>
 KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T, CB>& S, T* B = nullptr, int ldb = 0, int side_left = 0,
                      int nrhs = 0, T* Wt = nullptr)

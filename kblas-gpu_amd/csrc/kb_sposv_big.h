@@ -149,9 +149,24 @@ KB_DEV kb_f4 sb_clip(kb_f4 v, int row0, int n)
     return v;
 }
 
+// x + W (c - L x) for a diagonal tile: l and w are this lane's four elements of
+// the operands L and W (or their transposes), as in the sweeps.
+KB_DEV kb_f4 sb_correct(const float (&l)[4], const float (&w)[4], const kb_f4& c, kb_f4 x)
+{
+    kb_f4 r = c;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) r = mfma16x16x4(-l[s], x[s], r);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) x = mfma16x16x4(w[s], r[s], x);
+    return x;
+}
+
 // One wave: z := L^-1 z for 16 packed right-hand sides, left-looking by blocks
 // of SB_R tiles; W: the inverses of the diagonal tiles (16 x 16, row-major).
-// Sums of SB_KT tiles, as in ll_update.
+// Sums of SB_KT tiles, as in ll_update.  COR: the products with the inverses get
+// the correction of ll_solve (both sweeps); without it, a kernel matrix of
+// condition 5e12 took up to 19 refinement steps for 7, or none of 30 converged.
+template <bool COR>
 KB_DEV void sb_fwd(const float* L, int n, const float* W, float* z, int lane)
 {
     // formed here, not kept live across the phases of a matrix
@@ -225,6 +240,19 @@ KB_DEV void sb_fwd(const float* L, int n, const float* W, float* z, int lane)
                 x[r] = kb_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int s = 0; s < 4; ++s) x[r] = mfma16x16x4(w[r][s], c[r][s], x[r]);
+                if (COR) {
+                    const int c0 = 16 * (I + r), row = c0 + li;
+                    float l[4], wr[4];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const int col = c0 + 4 * lg + s;
+                        const bool in = row < n && col <= row;
+                        const float v = gld_opaque(L + (in ? row + (long)col * n : 0));
+                        l[s] = in ? v : 0.0f;
+                        wr[s] = w[r][s];
+                    }
+                    x[r] = sb_correct(l, wr, c[r], x[r]);
+                }
                 x[r] = sb_clip(x[r], 16 * (I + r) + 4 * lg, n);
                 gst((kb_f4*)(zl + (I + r) * 256L), x[r]);
             }
@@ -235,6 +263,7 @@ KB_DEV void sb_fwd(const float* L, int n, const float* W, float* z, int lane)
 // One wave: z := L^-T z, then X := (first ? 0 : X) + z for right-hand sides
 // 16 cb .. 16 cb + 15; returns the bits of max |x| over this lane's right-hand
 // side.
+template <bool COR>
 KB_DEV unsigned long long sb_bwd(const float* L, int n, const float* W, float* z, int lane, double* X, int ldx,
                                  int side_left, int nrhs, int cb, bool first)
 {
@@ -313,6 +342,17 @@ KB_DEV unsigned long long sb_bwd(const float* L, int n, const float* W, float* z
                 x[r] = kb_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int s = 0; s < 4; ++s) x[r] = mfma16x16x4(w[r][s], c[r][s], x[r]);
+                if (COR) {
+                    const int col = 16 * (I + r) + li;
+                    float l[4];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const bool in = row0 + s < n && col <= row0 + s;
+                        const float v = gld_opaque(L + (in ? row0 + s + (long)col * n : 0));
+                        l[s] = in ? v : 0.0f;
+                    }
+                    x[r] = sb_correct(l, w[r], c[r], x[r]);
+                }
                 x[r] = sb_clip(x[r], row0, n);
                 gst((kb_f4*)(zl + (I + r) * 256L), x[r]);
 #pragma unroll
@@ -511,12 +551,13 @@ KB_DEV void sb_sposv_one(long mat, int n, int nrhs, int side_left, double* Ap, i
     if (wave < ncb) sb_pack(Bp, ldb, side_left, n, nrhs, wave, z, big, lane);
     sb_convert(Ap, lda, n, A32, big);
     double cte = 0.0;
-    int iters = 0;
+    int iters = 0, cor = 0;
     bool ok = !__syncthreads_or(big);
     if (!ok) {
         iters = -2;
     } else {
         const int f32 = blk_potrf<float>(A32, n, n, S.f, nullptr, 0, 0, 0, W);
+        cor = uniform(S.f.grow) & KB_GROW_ANY;
         if (f32 != 0) {
             ok = false;
             iters = -3;
@@ -526,8 +567,15 @@ KB_DEV void sb_sposv_one(long mat, int n, int nrhs, int side_left, double* Ap, i
         // x += (L32 L32^T)^-1 r  (r = b at it = 0)
         if (threadIdx.x < KB_SB_MAX_RHS) S.rn[threadIdx.x] = 0ull;
         if (wave < ncb) {
-            sb_fwd(A32, n, W, z, lane);
-            const unsigned long long m = sb_lane_max(sb_bwd(A32, n, W, z, lane, Xp, ldx, side_left, nrhs, wave, it == 0));
+            unsigned long long m;
+            if (cor) {
+                sb_fwd<true>(A32, n, W, z, lane);
+                m = sb_bwd<true>(A32, n, W, z, lane, Xp, ldx, side_left, nrhs, wave, it == 0);
+            } else {
+                sb_fwd<false>(A32, n, W, z, lane);
+                m = sb_bwd<false>(A32, n, W, z, lane, Xp, ldx, side_left, nrhs, wave, it == 0);
+            }
+            m = sb_lane_max(m);
             if (lane < 16) S.xn[16 * wave + lane] = m;
         }
         __syncthreads();
