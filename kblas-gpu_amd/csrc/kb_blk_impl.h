@@ -738,7 +738,7 @@ KB_DEV int blk_potrf(T* A, int lda, int n, BlkSmem<T, CB>& S, T* B = nullptr, in
     asm volatile("" : "+v"(tid));   // lane-dependent values formed per call, not kept live across
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int li = lane & 15, lg = lane >> 4;
-    const int nrt = B ? (nrhs + 15) >> 4 : 0;
+    const int nrt = B ? (max(nrhs, 0) + 15) >> 4 : 0;   // (non-uniform counts come unchecked from the device)
     for (int k0 = 0; k0 < n; k0 += NBK) {
         const int kb = min(NBK, n - k0);
         const int nt = max((n - k0 - NBK + 15) >> 4, 0);   // row tiles below the diagonal block
