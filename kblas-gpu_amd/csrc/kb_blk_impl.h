@@ -187,14 +187,14 @@ KB_DEV void blk_diag_subst(T* B, int ldb, int side_left, int k0, int kb, int c0,
     }
 }
 
-// all rc right-hand sides of a pass of up to 16 CB
+// all rc right-hand sides of a pass of up to 16 CB (ncb blocks of 16)
 template <typename T, bool FWD, int CB, int W>
-KB_DEV void blk_diag_subst_n(T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T, CB>& S, T* sY,
+KB_DEV void blk_diag_subst_n(int ncb, T* B, int ldb, int side_left, int k0, int kb, int c0, int rc, BlkSmem<T, CB>& S, T* sY,
                              T sc = T(1))
 {
     constexpr int MX = 16 * CB / (W / 16);   // groups of a full pass
     static_assert(MX == 2 || MX == 4, "one case per group count");
-    const int ns = (rc + W / 16 - 1) / (W / 16);
+    const int ns = W == 256 ? ncb : (rc + W / 16 - 1) / (W / 16);
     if (MX == 2 || ns <= 2) {
         if (ns == 1) blk_diag_subst<T, 1, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
         else blk_diag_subst<T, 2, FWD, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
@@ -299,7 +299,7 @@ KB_DEV void blk_fwd_step(const T* L, int lda, int n, int k0, int kb, T* B, int l
     for (int c0 = 0; c0 < nrhs; c0 += RC) {
         const int rc = min(RC, nrhs - c0);
         const int ncb = (rc + 15) / 16;
-        blk_diag_subst_n<T, true, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+        blk_diag_subst_n<T, true, CB, W>(ncb, B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
         __syncthreads();
         blk_update_rows_n<T, false, CB, W>(ncb, L, lda, B, ldb, side_left, k0, kb, k0 + kb, n, c0, rc, sY, sc);
         __syncthreads();
@@ -344,7 +344,7 @@ KB_DEV void blk_solve_bwd(const T* L, int lda, int n, T* B, int ldb, int side_le
         for (int c0 = 0; c0 < nrhs; c0 += RC) {
             const int rc = min(RC, nrhs - c0);
             const int ncb = (rc + 15) / 16;
-            blk_diag_subst_n<T, false, CB, W>(B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
+            blk_diag_subst_n<T, false, CB, W>(ncb, B, ldb, side_left, k0, kb, c0, rc, S, sY, sc);
             __syncthreads();
             blk_update_rows_n<T, true, CB, W>(ncb, L, lda, B, ldb, side_left, k0, kb, 0, k0, c0, rc, sY, sc);
             __syncthreads();
