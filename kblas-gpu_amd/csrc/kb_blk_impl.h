@@ -829,29 +829,59 @@ k_blk_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* in
 
 // Passes of 32 right-hand sides when the count allows (POTRF: none), else 64.
 constexpr int KB_BLK_NARROW = 32;
+// Matrices the 256-thread kernel holds at once (256 CUs; registers allow four,
+// five or six workgroups).
+template <typename T, int MODE> constexpr int blk_held()
+{
+    if (MODE == KB_MODE_POTRS) return 256 * (sizeof(T) == 8 ? 5 : 6);
+    return 256 * (sizeof(T) == 4 && MODE == KB_MODE_POTRF ? 5 : 4);
+}
+
 // Two waves per matrix instead of four where a panel has too few row tiles to
 // keep three waves busy while the first factors the diagonal block: twice the
-// matrices per CU then hide its chain.  Only for batches that fill the chip with
-// four waves each (256 CUs x 4 workgroups), and up to the order, or order and
-// right-hand sides, where the four waves' updates win again.  256 -> 128
-// threads (us, with the copies that restore the inputs): DPOTRF n = 80 x 10,000
-// 546 -> 448, n = 200 x 2,000 585 -> 560, n = 256 x 4,096 1,762 -> 1,810; DPOSV n
-// = 100 x 5,000, 8 right-hand sides 611 -> 505, n = 200 x 3,000, 4 right-hand
-// sides 1,088 -> 1,058, 30 right-hand sides 1,340 -> 1,433; DPOTRS n = 224 x
-// 1,100, 16 right-hand sides 192 -> 213.
-constexpr int KB_BLK_FULL = 1024;
+// matrices per CU then hide its chain.  Only for batches that the four-wave form
+// does not hold at once, and up to the order and right-hand sides where the four
+// waves' updates win again (POTRS beyond 2,048 matrices: earlier, the factors in
+// flight, read twice, no longer fit the caches).  256 -> 128 threads, us: DPOTRF n = 80 x
+// 4,000 152 -> 101, n = 200 x 1,300 to 4,000 0.95 to 1.04 of the time; SPOTRF n = 128 x
+// 1,100 53 -> 57, x 1,300 79 -> 59; SPOSV n = 128 x 2,100, 8 right-hand sides 185 ->
+// 151; DPOTRS n = 192 x 4,000, 8 right-hand sides 434 -> 394, n = 130, 16 right-hand
+// sides, x 1,700 0.98 of the time, x 2,100 156 -> 184; SPOTRS n = 100 x 1,300, 17
+// right-hand sides 77 -> 85, x 1,700 0.93 of the time.
+template <typename T, int MODE>
+static bool blk_two_waves(int n, int nrhs, int batch)
+{
+    int nmax = 224;
+    if (MODE != KB_MODE_POTRF && nrhs > 4) nmax = nrhs <= 16 ? 192 : 128;
+    if (MODE == KB_MODE_POTRS && nrhs > 8 && batch > 2048) nmax = nrhs <= 24 ? 128 : 96;
+    return n <= nmax && batch > blk_held<T, MODE>();
+}
+
+// FP64 POTRS: dynamic LDS that leaves four of five workgroups to a CU, where the
+// fifth saves no round or is one of many: it only pushes the factors, read twice,
+// out of the caches (n = 200 x 1,300, 32 right-hand sides 385 us, with four 363).
+template <typename T, int MODE>
+static int blk_pad_lds(int nrhs, int batch)
+{
+    const bool pad = sizeof(T) == 8 && MODE == KB_MODE_POTRS && nrhs > 8 &&
+                     (batch > 2 * 1280 || (batch + 1023) / 1024 == (batch + 1279) / 1280);
+    return pad ? 16384 : 0;
+}
 
 template <typename T, int MODE>
 static void launch_blk_mode(int n, int nrhs, int side_left, BatchArg<T> a, BatchArg<T> b, int* info, int batch,
                             int grid, hipStream_t s)
 {
     const bool narrow = MODE == KB_MODE_POTRF || nrhs <= KB_BLK_NARROW;
-    if (narrow && batch > KB_BLK_FULL && n <= (MODE == KB_MODE_POTRF || nrhs <= 4 ? 224 : nrhs <= 16 ? 192 : 128))
-        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, 128>), dim3(grid), dim3(128), 0, s, n, nrhs, side_left, a, b, info,
-                           batch);
+    if (narrow && blk_two_waves<T, MODE>(n, nrhs, batch))
+        // (a CU holds eight, in FP32 POTRS fourteen: n = 128 x 2,100, 8 right-hand
+        // sides 1.04 of the four waves' time with 2,048 workgroups, 0.90 with more)
+        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, 128>),
+                           dim3(sizeof(T) == 4 && MODE == KB_MODE_POTRS ? min(batch, 4096) : grid), dim3(128), 0, s, n,
+                           nrhs, side_left, a, b, info, batch);
     else if (narrow)
-        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, KB_BLK_WG>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a,
-                           b, info, batch);
+        hipLaunchKernelGGL((k_blk_chol<T, MODE, 2, KB_BLK_WG>), dim3(grid), dim3(KB_BLK_WG),
+                           (blk_pad_lds<T, MODE>(nrhs, batch)), s, n, nrhs, side_left, a, b, info, batch);
     else
         hipLaunchKernelGGL((k_blk_chol<T, MODE, 4, KB_BLK_WG>), dim3(grid), dim3(KB_BLK_WG), 0, s, n, nrhs, side_left, a,
                            b, info, batch);
