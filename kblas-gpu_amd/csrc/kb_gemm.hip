@@ -365,15 +365,21 @@ int gm_dispatch(int ta, int tb, int m, int n, int k, T alpha, kb_mat_t A, kb_mat
     if (m <= 16 || n <= 16) return gm_trans<T, 16>(ta, tb, m, n, k, alpha, A, B, beta, C,
         batch, syrk, upper, vm, vn, vk, skip, s);
     // SYRK on the workgroup tiles where their padding to 64 costs nothing over the
-    // wavefront tiles' padding to 32 (an even number of 32s): with an odd one they
-    // do 1.3 to 1.7 times the products.  Batch of 2,000 to 20,000, wavefront ->
-    // workgroup tiles, FP32: n = 64 274 -> 237 us, n = 100, k = 30 242 -> 194, n =
-    // 256, k = 16 273 -> 178, k = 256 731 -> 621, but n = 96 265 -> 310; FP64, bound
-    // by the matrix cores either way: n = 256 1,057 -> 1,014 but n = 64 364 -> 394,
-    // n = 128 714 -> 705.  (Non-uniform batches keep the wavefront tiles: their
+    // wavefront tiles' padding to 32 (an even number of 32s; with an odd one they do
+    // 1.3 to 1.7 times the products: n = 96 265 -> 310 us) and enough of them are in
+    // flight to hide a chunk's barrier.  Wavefront -> workgroup tiles, us:
+    // FP32 n = 256 x 1,000, k = 16 98 -> 63, k = 256 349 -> 292; x 16 (160 tiles) k = 16
+    // 9.8 -> 9.2, k = 256 18.4 -> 22.6, x 64 1.00 and x 150 0.84 of the time; n = 64,
+    // k = 64, x 600 1.18, x 1,000 1.08, x 2,000 0.90.  FP64, bound by the matrix cores
+    // either way: n = 256 x 1,000, k = 16 154 -> 169, k = 32 175 -> 183, k = 64 217 -> 214,
+    // k = 256 502 -> 483; x 16, k = 256 23.2 -> 24.4;
+    // n = 64 x 10,000 364 -> 394.  (Non-uniform batches keep the wavefront tiles: their
     // orders differ from the bound.)
     const bool even = (((m + 31) / 32) & 1) == 0;
-    const bool sy_lds = !vm && even && m >= GM_LDS_MIN && (sizeof(T) == 4 || m > 192);
+    const long t64 = (m + GL_TM - 1) / GL_TM, sy_tiles = batch * (t64 * (t64 + 1) / 2);
+    const bool sy_fill = sizeof(T) == 4 ? k <= 16 || sy_tiles >= (m <= 128 ? 1536 : 640)
+                                        : m > 192 && k >= 48 && sy_tiles >= 512;
+    const bool sy_lds = !vm && even && m >= GM_LDS_MIN && sy_fill;
     if ((syrk && !sy_lds) || m < GM_LDS_MIN || n < GM_LDS_MIN)
         return gm_trans<T, 32>(ta, tb, m, n, k, alpha, A, B, beta, C, batch, syrk, upper, vm, vn, vk, skip, s);
     return gm_trans<T, GL_TM>(ta, tb, m, n, k, alpha, A, B, beta, C, batch, syrk, upper, vm, vn, vk, skip, s);
