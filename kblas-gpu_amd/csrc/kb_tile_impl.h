@@ -347,12 +347,13 @@ KB_DEV void tile_chol_one(int n, int nrhs, int side_left, T* Ap, int lda, T* Bp,
     int inf = 0;
     const int i = lane & 15;
     typename TileV<T>::v4 t[10];
-    // the first right-hand sides go out with the matrix: one wait for memory
+    // POTRS in passes of eight: the first right-hand sides go out with the matrix, one
+    // wait for memory (SPOTRS n = 64 x 20,000, 8 right-hand sides 108 -> 91 us).  Passes
+    // of four gain nothing, and POSV would hold them through the factorization (SPOSV
+    // n = 64 x 100, one right-hand side 23.0 -> 24.2 us, eight 24.8 -> 26.1).
+    constexpr bool EARLY = MODE == KB_MODE_POTRS && NG > 1;
     T v[NG][4];
-    if constexpr (MODE != KB_MODE_POTRF) {
-        // (POSV without right-hand sides only factors: B may not exist)
-        if (nrhs > 0) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, 0, lane);
-    }
+    if constexpr (EARLY) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, 0, lane);
     if constexpr (MODE != KB_MODE_POTRS) {
         tile_load<T>(t, Ap, lda, n, lane);
         inf = tile_potrf<T>(t, invd, n, S.pan, lane);
@@ -372,7 +373,7 @@ KB_DEV void tile_chol_one(int n, int nrhs, int side_left, T* Ap, int lda, T* Bp,
 #pragma unroll
         for (int K = 0; K < 4; ++K) S.invd[K][lane] = invd[K];
         for (int c0 = 0; c0 < nrhs; c0 += 4 * NG) {
-            if (c0 > 0) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, c0, lane);
+            if (!EARLY || c0 > 0) tile_rhs<T, NG>(v, Bp, ldb, side_left, n, nrhs, c0, lane);
 #pragma unroll
             for (int q = 0; q < NG; ++q)
 #pragma unroll
