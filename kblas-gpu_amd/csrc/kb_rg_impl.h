@@ -209,7 +209,9 @@ KB_DEV void rg_rhs(T (&x)[RC][NB / 16], T* Bp, int ldb, int side_left, int n, in
 // ---------------------------------------------------------------------------
 // one matrix per 16-lane row; WPB wavefronts (4 WPB matrices) per workgroup
 // ---------------------------------------------------------------------------
-template <typename T, int NB, int MODE, int RC, bool EX, int WPB>
+// EARLY (POTRS): the first right-hand sides go out with the factor, so the call
+// waits for memory once (POSV's registers are full during the factorization).
+template <typename T, int NB, int MODE, int RC, bool EX, int WPB, bool EARLY = MODE == KB_MODE_POTRS>
 __global__ void __launch_bounds__(64 * WPB)
 k_rg_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* info, int batch)
 {
@@ -233,9 +235,6 @@ k_rg_chol(int n, int nrhs, int side_left, BatchArg<T> A, BatchArg<T> B, int* inf
 #pragma unroll
     for (int s = 0; s < R; ++s) dinv2[s] = T(1);
     rg_load<T, NB, EX>(a, Ap, lda, n, l);
-    // POTRS: the first right-hand sides go out with the factor, so the call waits
-    // for memory once (POSV's registers are full during the factorization)
-    constexpr bool EARLY = MODE == KB_MODE_POTRS;
     T x0[EARLY ? RC : 1][R];
     if constexpr (EARLY) rg_rhs<T, NB, RC, EX>(x0, B.get(m), B.ldim(m), side_left, n, nrhs, 0, l);
 
