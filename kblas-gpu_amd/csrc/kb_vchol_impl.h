@@ -249,8 +249,12 @@ static int launch_vchol(const int* vm, const int* vn, int side_left, kb_mat_t A,
         hipLaunchKernelGGL((k_vchol_blk<T, MODE, 2>), dim3(vchol_grid(k_vchol_blk<T, MODE, 2>, batch)),
                            dim3(KB_BLK_WG), 0, s, vm, vn, side_left, a, b, x, info, iter, batch, ws);
     else
+        // POTRS: dynamic LDS that leaves three of four workgroups to a CU, as the
+        // fourth only pushes the factors, read twice, out of the caches (orders
+        // 65..512 x 1,000, 64 right-hand sides: four 1.14 ms, three 1.08)
         hipLaunchKernelGGL((k_vchol_blk<T, MODE, 4>), dim3(vchol_grid(k_vchol_blk<T, MODE, 4>, batch)),
-                           dim3(KB_BLK_WG), 0, s, vm, vn, side_left, a, b, x, info, iter, batch, ws);
+                           dim3(KB_BLK_WG), sizeof(T) == 8 && MODE == KB_MODE_POTRS ? 16384 : 0, s, vm, vn, side_left,
+                           a, b, x, info, iter, batch, ws);
     hipLaunchKernelGGL((k_vchol_small<T, MODE>), dim3(vchol_grid(k_vchol_small<T, MODE>, (batch + 3) / 4)),
                        dim3(KB_BLK_WG), 0, s, vm, vn, side_left, a, b, x, info, iter, batch, ws);
     return (int)hipGetLastError();
