@@ -246,7 +246,11 @@ k_inv_reg(int op, int unit, int n, BatchArg<T> A, int* info, const int* skip, in
 // sum_k U(a,k) U(c,k) over k ascending, with U(c,k) from lane c the same way.  No
 // LDS: the register form above is bound by its LDS broadcasts (every lane reads
 // the whole triangle twice).  POTRI n = 32 x 10,000 FP64: 65 -> 34 us,
-// POTI with the factorization before it 82 -> 51 us; n = 16 x 20,000 24 -> 13 us.
+// POTI with the factorization before it 82 -> 54 us; n = 16 x 20,000 24 -> 13 us.
+// Row a also multiplies elements by its zeros left of the diagonal, so an infinity
+// or a NaN in L would reach results that do not depend on it.  Such an element
+// always leaves some row's last column not finite; that matrix is then computed by
+// the loops of the larger orders (inv_run) instead.
 template <int NB, typename T>
 __global__ void __launch_bounds__(64)
 k_potri_dpp(int n, BatchArg<T> A, int* info, const int* skip, int batch)
@@ -298,8 +302,12 @@ k_potri_dpp(int n, BatchArg<T> A, int* info, const int* skip, int batch)
             }
         }
     }
+    bool fin = true;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) fin = fin && kb_abs<T>(x[s][NB - 1]) < T(__builtin_inf());
+    const unsigned long long odd = __ballot(!fin);   // (by rows of 16: one per matrix)
     // rows of the result, a column at a time
-    const bool wr = live && inf == 0;
+    const bool wr = live && inf == 0 && ((odd >> (lane & 48)) & 0xffffu) == 0;
     T* q = G + i;
 #pragma unroll
     for (int c = 0; c < NB; ++c) {
@@ -319,6 +327,15 @@ k_potri_dpp(int n, BatchArg<T> A, int* info, const int* skip, int batch)
         asm volatile("" : "+v"(q));
     }
     if (live && info && i == 0) info[b] = inf <= n ? inf : 0;
+    if (odd) {
+        __shared__ int sflag;
+        for (int g = 0; g < 4; ++g) {
+            const long bg = (long)blockIdx.x * 4 + g;
+            if (((odd >> (16 * g)) & 0xffffu) == 0 || bg >= batch || (skip && skip[bg] != 0)) continue;
+            inv_run<T>(KB_INV_OP_POTRI, 0, A.get(bg), A.ldim(bg), n, lane, &sflag);   // (not with a zero pivot)
+            __syncthreads();
+        }
+    }
 }
 
 // ---------------------------------------------------------------- TRMM ----
