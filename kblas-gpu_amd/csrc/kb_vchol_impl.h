@@ -160,35 +160,19 @@ k_vchol_blk(const int* vm, const int* vn, int side_left, BatchArg<T> A, BatchArg
         const long mat = uniform(q.order[ticket]);
         const int n = uniform(vq_order(vm, vn, side_left, mat));
         const int nrhs = uniform(vq_nrhs(vm, vn, side_left, mat));
-        if constexpr (MODE == KB_MODE_SPOSV) {
-            // Orders above the register range are solved in FP64 directly
-            // (LAPACK dsposv's ITER = -1: full precision for implementation
-            // reasons); A receives L as in the dsposv fallback.
-            T* Ap = uniform(A.get(mat));
-            const int lda = uniform(A.ldim(mat));
+        T* Ap = uniform(A.get(mat));
+        const int lda = uniform(A.ldim(mat));
+        if constexpr (MODE == KB_MODE_POTRF) {
+            const int inf = blk_potrf<T, CB>(Ap, lda, n, S);
+            if (threadIdx.x == 0 && info) info[mat] = inf;
+        } else if constexpr (MODE == KB_MODE_POSV) {
             T* Bp = uniform(B.get(mat));
-            T* Xp = uniform(X.get(mat));
-            const int ldb = uniform(B.ldim(mat)), ldx = uniform(X.ldim(mat));
-            copy_rhs<T>(Bp, ldb, Xp, ldx, side_left, n, nrhs, threadIdx.x, KB_BLK_WG);
-            __syncthreads();
-            const int inf = blk_potrf<T, CB>(Ap, lda, n, S, Xp, ldx, side_left, nrhs);
-            if (threadIdx.x == 0) { if (info) info[mat] = inf; if (iter) iter[mat] = -1; }
-            if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Xp, ldx, side_left, nrhs, S);
+            const int ldb = uniform(B.ldim(mat));
+            const int inf = blk_potrf<T, CB>(Ap, lda, n, S, Bp, ldb, side_left, nrhs);
+            if (threadIdx.x == 0 && info) info[mat] = inf;
+            if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Bp, ldb, side_left, nrhs, S);
         } else {
-            T* Ap = uniform(A.get(mat));
-            const int lda = uniform(A.ldim(mat));
-            if constexpr (MODE == KB_MODE_POTRF) {
-                const int inf = blk_potrf<T, CB>(Ap, lda, n, S);
-                if (threadIdx.x == 0 && info) info[mat] = inf;
-            } else if constexpr (MODE == KB_MODE_POSV) {
-                T* Bp = uniform(B.get(mat));
-                const int ldb = uniform(B.ldim(mat));
-                const int inf = blk_potrf<T, CB>(Ap, lda, n, S, Bp, ldb, side_left, nrhs);
-                if (threadIdx.x == 0 && info) info[mat] = inf;
-                if (inf == 0) blk_solve_bwd<T, CB>(Ap, lda, n, Bp, ldb, side_left, nrhs, S);
-            } else {
-                blk_solve<T, CB>(Ap, lda, n, uniform(B.get(mat)), uniform(B.ldim(mat)), side_left, nrhs, S);
-            }
+            blk_solve<T, CB>(Ap, lda, n, uniform(B.get(mat)), uniform(B.ldim(mat)), side_left, nrhs, S);
         }
         __syncthreads();
     }
