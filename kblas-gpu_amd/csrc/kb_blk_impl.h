@@ -382,13 +382,14 @@ constexpr int KB_LL_U = 1;
 constexpr int KB_LL_KC = 64;   // columns whose products are summed before they are taken from C
 
 // A diagonal tile L counts as ill-conditioned when four columns of W = L^-1 give a
-// row of |W| |L| (unchanged by a scaling of A's rows and columns) more than this,
-// or a NaN; its row sums stay below 16 otherwise.  B B^T + n I of order 200 has
-// sums of 1.6, Q diag(s) Q^T of condition 1e4 up to 10, a Gaussian kernel matrix
-// at the limit of FP64 1e6: without the correction POTRF's error there is 1,000
-// times substitution's, or a pivot comes out negative.  Forming the measure is in
-// wave 0's serial part: DPOTRF n = 200, one matrix, 87.7 -> 88.7 us, SPOTRF 66.9 ->
-// 68.3 us, batches that fill the chip as before.
+// row of |W| |L| (unchanged by a scaling of A's rows and columns) more than this;
+// its row sums stay below 16 otherwise.  B B^T + n I of order 200 has sums of 1.6,
+// Q diag(s) Q^T of condition 1e4 up to 10, a Gaussian kernel matrix at the limit of
+// FP64 1e6: without the correction POTRF's error there is 1,000 times
+// substitution's, or a pivot comes out negative.  (Not with a NaN in |W| |L|: an
+// infinity on A's diagonal leaves a zero column in W, and c - L x would be NaN.)
+// Forming the measure is in wave 0's serial part: DPOTRF n = 200, one matrix, 87.7
+// -> 88.7 us, SPOTRF 66.9 -> 68.3 us, batches that fill the chip as before.
 constexpr int KB_LL_GROW = 4;
 // The same for the mixed routine's FP32 sweeps, whose result a refinement corrects:
 // row sums below 128 cost no more than the rounding of a substitution over 65 or
@@ -701,21 +702,23 @@ KB_DEV void ll_diag(T* A, int lda, int k0, int kb, BlkSmem<T, CB>& S, int lane, 
             for (int s = 0; s < 4; ++s) fnmac_rowk<T>(y[b][s], y[b][s] * ij, l, j);
         }
     }
-    int grow = k0 > 0 ? S.grow & KB_GROW_ANY : 0;
+    T m[2];   // this lane's four columns' part of a row of |W| |L| (its sum)
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
-        T m = T(0);   // this lane's four columns' part of a row of |W| |L| (its sum)
+        m[b] = T(0);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const T v = y[b][s] * S.sInv[16 * b + i];
             S.fW[b][i * KB_LL_LD + 4 * g + s] = v;
             if (W && 16 * b < kb) gst(W + 16L * (k0 + 16 * b) + 16 * i + 4 * g + s, v);
-            m += kb_abs<T>(v) * lsum[b][s];
+            m[b] += kb_abs<T>(v) * lsum[b][s];
         }
-        if (__any(!(m <= T(KB_LL_GROW)))) {
-            grow |= KB_GROW_NOW;
-            if (__any(!(m <= T(KB_LL_GROW_SWEEP)))) grow |= KB_GROW_ANY;
-        }
+    }
+    int grow = k0 > 0 ? S.grow & KB_GROW_ANY : 0;
+    const T mm = m[0] > m[1] ? m[0] : m[1], ms = m[0] + m[1];
+    if (__any(mm > T(KB_LL_GROW)) && !__any(ms != ms)) {
+        grow |= KB_GROW_NOW;
+        if (__any(mm > T(KB_LL_GROW_SWEEP))) grow |= KB_GROW_ANY;
     }
     if (lane == 0) S.grow = grow;
 }
