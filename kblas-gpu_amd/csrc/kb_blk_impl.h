@@ -1,5 +1,6 @@
-// kb_blk_impl.h -- blocked batched Cholesky family, one 256-thread workgroup
-// per matrix, for orders above the register-resident range.
+// kb_blk_impl.h -- blocked batched Cholesky family, one workgroup per matrix (four
+// waves, two for large batches of smaller orders), for orders above the
+// register-resident range.
 //
 // Left-looking blocked algorithm with panel width NBK = 32, the same POTRF ->
 // TRSM(R,L,T) -> SYRK(L,N,-1,+1) arithmetic the reference runs as a recursion
@@ -9,20 +10,22 @@
 //     the products of the finished columns on the matrix cores, factors it in
 //     registers (4-column panels on DPP rows, rank-4 updates on the matrix
 //     cores) and leaves the inverses of the two 16x16 diagonal tiles in LDS;
-//   - meanwhile waves 1..3 read the 16-row tiles below and subtract the same
+//   - meanwhile the other waves read the 16-row tiles below and subtract the same
 //     products, then solve them against the inverses (with a correction step
 //     where a diagonal tile is ill-conditioned), all in registers: every
 //     element of A is read once and every element of L written once, and the
 //     only other traffic is re-reading finished columns of L;
 //   - right-hand sides (POSV) are further row tiles of the panel: the forward
 //     sweep L Y = B is the panel solve Y^T = B^T L^-T.
-// What bounds it: the serial chain of a panel (the loads' latency, the 32
-// pivots, two barriers), hidden by the four or eight workgroups of a CU.  Against
-// the right-looking form it replaces (trailing matrix read and written once per
-// 64 columns, rows solved by substitution one per thread): DPOTRF n = 200 x
-// 2,000 725 -> 300 us, n = 256 x 4,096 1.82 -> 0.85 ms, n = 128 x 8,000 0.82 ->
-// 0.32 ms; the workgroup phase of the non-uniform DPOSV of orders 8..256 x
-// 20,000 4.69 -> 2.82 ms.
+// What bounds it: for small batches the serial chain of a panel (the loads'
+// latency, the 32 pivots, two barriers); with the four or eight workgroups of a CU
+// that hide it, memory (finished columns are read again once per panel: the
+// non-uniform DPOSV of orders 8..256 moves 13.1 GB in 2.82 ms, a copy's rate).
+// Against the right-looking form it replaces (trailing matrix read and written once
+// per 64 columns, rows solved by substitution one per thread), kernel times: DPOTRF
+// n = 200 x 2,000 721 -> 339 us, n = 256 x 4,096 1.82 -> 0.92 ms, n = 128 x 8,000 0.86 ->
+// 0.37 ms; SPOTRF n = 200 x 4,000 966 -> 397 us; the workgroup phase of the non-uniform
+// DPOSV of orders 8..256 x 20,000 4.69 -> 2.82 ms.
 // The solve (POSV/POTRS) runs blocked forward and backward sweeps over up to
 // 64 right-hand sides per pass (so L is streamed once per sweep for up to 64
 // right-hand sides): the diagonal blocks by DPP-row substitutions, the
@@ -38,9 +41,8 @@ constexpr int KB_BLK_NBK = 32;
 constexpr int KB_BLK_WG = 256;
 constexpr int KB_LL_LD = 17;    // pitch of a staged 16 x 16 tile
 // 16-row tiles a wave holds at once (C and the running sums: FP64 16 VGPRs each
-// per tile).  FP64: 2 fill the 128 VGPRs that four workgroups per CU leave; 3
-// spill there, and with three workgroups per CU n = 128 takes 0.61 instead of
-// 0.45 ms.  FP32: 4 against 2 is n = 200 x 4,000 0.57 against 0.63 ms.
+// per tile), kernel times: FP64 2 against 3, n = 128 x 8,000 373 against 363 us, n =
+// 128 x 1,000 64.4 against 65.6; FP32 4 against 2, n = 200 x 4,000 397 against 431 us.
 template <typename T> constexpr int ll_g();
 template <> constexpr int ll_g<double>() { return 2; }
 template <> constexpr int ll_g<float>() { return 4; }

@@ -36,8 +36,8 @@ constexpr int KB_SB_ITERMAX = 30;
 
 struct SbSmem {
     union {
-        BlkSmem<float> f;                  // FP32 factorization and solves
-        BlkSmem<double> d;                 // residual staging, FP64 path
+        BlkSmem<float> f;                  // FP32 factorization
+        BlkSmem<double> d;                 // FP64 path
     };
     unsigned long long rn[KB_SB_MAX_RHS];  // max |r| per right-hand side (bits of a non-negative double)
     unsigned long long xn[KB_SB_MAX_RHS];  // max |x| per right-hand side
